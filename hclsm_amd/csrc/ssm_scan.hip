@@ -16,29 +16,9 @@
 // run on the matrix core instead (ssm_scan_fwd_mfma_kernel below), which leaves
 // mul, exp, mul, fma per state update on the VALU.
 #include "internal.h"
+#include "scan_common.h"
 
 namespace hclsm {
-
-// Internal mode of hclsm_ssm_block_scan_fwd: the MODEL clamps, dt = softplus(dt input) before
-// its clamp, and the output multiplied by silu(gate) -- the SimplifiedSSMBlock epilogues
-// (level0_ssm.py:73, :76, :103) fused into the scan.
-constexpr int SCAN_BLOCK = HCLSM_SCAN_BLOCK;
-struct ScanEpi {
-  const void* gate;   // [batch][T][d_inner], I/O type; required in SCAN_BLOCK
-  void* y_pre;        // optional: the scan output before gating (kept for the backward)
-  float* ck;          // checkpointing launches only: [batch][ceil(T / 8)][16][d_inner] fp32, the state
-                      // before steps 8, 16, ... (the backward's checkpoint slab; entry 0, the zero initial
-                      // state, is not stored)
-};
-
-
-template <int MODE>
-__device__ __forceinline__ float scan_dt(float v) {
-  if constexpr (MODE == SCAN_BLOCK) v = softplus_f(v);
-  if constexpr (MODE != HCLSM_SCAN_RAW) v = fminf(fmaxf(v, 1e-3f), 1.0f);
-  return v;
-}
-
 
 constexpr int SCAN_TCHUNK = 8;
 constexpr int SCAN_MAX_BLOCK = 256;
@@ -783,6 +763,10 @@ static int scan_entry(int mode, const void* x, const void* dt, const float* A_lo
     return 0;
   }
   if (!x || !dt || !A_log || !B || !C || !y) return HCLSM_ERR_NULL;
+  {   // wide states (and small grids of d_state 16); the generic kernel takes what it refuses
+    const int r = scan_fwd_group(mode, x, dt, A_log, B, C, Dskip, y, h_final, batch, T, d_inner, d_state, dtype, st, epi);
+    if (r != HCLSM_ERR_UNSUPPORTED) return r;
+  }
   switch (dtype) {
     case HCLSM_F32:
       return dispatch_sp<HCLSM_F32>(mode, x, dt, A_log, B, C, Dskip, y, h_final, batch, T, d_inner, d_state, st, epi);
