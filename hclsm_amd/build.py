@@ -34,6 +34,7 @@ HIPCC_FLAGS = [
 FILE_FLAGS = {
     "ssm_scan.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ssm_scan_group.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "ssm_scan_bwd_group.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # The attention's score and output tiles are consumed by VALU code right after each MFMA; in the VGPR
     # form they need no AGPR copies and the kernel takes fewer registers (more waves per SIMD).
     "event_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

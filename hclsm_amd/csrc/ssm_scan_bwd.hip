@@ -8,6 +8,7 @@
 //   gA[d,s] = sum_{n,t} g_arg dt   with g_arg = gh_t h_{t-1} exp(dt A)
 // (model mode: each clamp passes gradient only inside its closed interval).
 //
+// fp32 and bf16 with d_state 24, 32, ... run in ssm_scan_bwd_group.hip; here d_state up to 16, fp16 and odd states.
 // Mapping: one lane owns channel d of sequence n and SG <= 16 of its states (G = d_state/SG lanes
 // per channel, adjacent); a workgroup holds up to 384 lanes of one sequence's channels.  Pass 1
 // recomputes h forward and writes the state at every chunk start (chunks of K = 32/SG steps) to a
@@ -18,6 +19,8 @@
 // followed by a cross-wave sum through LDS once per chunk, one part per channel block.  One tail launch
 // then reduces the per-sequence partials of gA_log and gD, and adds the blocks' gB / gC parts and casts.
 #include "internal.h"
+#include "ssm_scan_bwd_common.h"
+#include "ssm_scan_bwd_group.h"
 
 namespace hclsm {
 
@@ -37,42 +40,6 @@ static inline BwdGrid bwd_grid(int64_t Dn, int G) {
   return BwdGrid{(int)((Dn + nb - 1) / nb), (int)nb};
 }
 
-// Value of the partner lane across bit M for the reduce-scatter steps below 16 lanes.  The partner only
-// has to differ in bit M and agree in the bits above it; when every bit below M is reduced later too
-// (MASK_LO == 1) the DPP mirrors are used (lane ^ 15, lane ^ 7 inside a row), else exact xor partners.
-template <int M, int MASK_LO>
-__device__ __forceinline__ float rs_partner(float v) {
-  const int b = __float_as_int(v);
-  if constexpr (M == 8) {
-    return __int_as_float(MASK_LO == 1 ? __builtin_amdgcn_update_dpp(0, b, 0x140, 0xf, 0xf, true)     // row_mirror
-                                       : __builtin_amdgcn_update_dpp(0, b, 0x128, 0xf, 0xf, true));   // row_ror:8
-  } else if constexpr (M == 4) {
-    if constexpr (MASK_LO == 1)
-      return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x141, 0xf, 0xf, true));   // row_half_mirror
-    else
-      return __shfl_xor(v, 4, 64);
-  } else if constexpr (M == 2) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x4e, 0xf, 0xf, true));      // quad_perm 2,3,0,1
-  } else {
-    static_assert(M == 1, "rs_partner: M in {1, 2, 4, 8}");
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0xb1, 0xf, 0xf, true));      // quad_perm 1,0,3,2
-  }
-}
-
-// (lo, hi) -> lo summed over the lane pair for the lower lane, hi summed for the upper lane, where the
-// pair differs in bit 5 (M == 32) or bit 4 (M == 16): one gfx950 permlane swap exchanges the halves.
-template <int M>
-__device__ __forceinline__ float rs_swap_sum(float lo, float hi) {
-  if constexpr (M == 32) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  } else {
-    static_assert(M == 16, "rs_swap_sum: M in {16, 32}");
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-}
-
 // Sum over the G adjacent lanes of a channel (G a power of two <= 8), every lane gets the total.
 template <int G>
 __device__ __forceinline__ float group_sum(float v) {
@@ -82,46 +49,6 @@ __device__ __forceinline__ float group_sum(float v) {
   static_assert(G <= 8, "group_sum: at most 8 lanes");
   return v;
 }
-
-template <int V, int MASK_LO>
-struct RS {
-  // Reduce-scatter V values across the lanes that differ in bits [MASK_LO, 32] of the lane id.
-  // On return v[0 .. V/2^h) holds sums for value indices starting at `off` (h = halving steps).
-  template <int CNT, int M>
-  static __device__ __forceinline__ void step(float* v, int lane, int& off) {
-    if constexpr (M >= MASK_LO) {
-      if constexpr (CNT > 1) {
-        const bool upper = (lane & M) != 0;
-#pragma unroll
-        for (int i = 0; i < CNT / 2; ++i) {
-          if constexpr (M >= 16) {
-            v[i] = rs_swap_sum<M>(v[i], v[i + CNT / 2]);
-          } else {
-            const float keep = upper ? v[i + CNT / 2] : v[i];
-            const float send = upper ? v[i] : v[i + CNT / 2];
-            v[i] = keep + rs_partner<M, MASK_LO>(send);
-          }
-        }
-        if (upper) off += CNT / 2;
-        step<CNT / 2, M / 2>(v, lane, off);
-      } else {
-        if constexpr (M >= 16) v[0] = rs_swap_sum<M>(v[0], v[0]);
-        else v[0] += rs_partner<M, MASK_LO>(v[0]);
-        step<1, M / 2>(v, lane, off);
-      }
-    }
-  }
-  static __device__ __forceinline__ int run(float* v, int lane) {
-    int off = 0;
-    step<V, 32>(v, lane, off);
-    return off;
-  }
-};
-
-template <int N_, int MASK_LO> struct RSCount {  // values left per lane after RS
-  static constexpr int h(int cnt, int m) { return (m < MASK_LO || cnt <= 1) ? cnt : h(cnt / 2, m / 2); }
-  static constexpr int value = h(N_, 32);
-};
 
 struct BwdArgs {
   int T, Dn, S, nchunk, nck, DW;   // nck = checkpoints per sequence = ceil(nchunk / BWD_CKR)
@@ -390,15 +317,15 @@ ssm_scan_bwd_kernel(const typename Elem<DT>::T* __restrict__ x, const typename E
 }
 
 // The backward's tail in one launch: blocks [0, nga) reduce the per-sequence gA partials over the sequences and
-// write gA_log[d, s] = sum * dA/dA_log; blocks [nga, nga + ngd) reduce the gD partials; the remaining blocks add
+// write gA_log[d, s] = sum * dA/dA_log (SP: states per channel in the partials, S of them real); blocks [nga, nga + ngd) reduce the gD partials; the remaining blocks add
 // the channel blocks' gB / gC parts in block order and cast.  The three parts are independent.  Each reducing
 // block sums 64 columns in 16 row groups (fixed order: deterministic).
-template <int DT, int SP, int MODE>
+template <int DT, int MODE>
 __global__ void __launch_bounds__(1024)
 ssm_scan_bwd_tail(const float* __restrict__ ga_part, const float* __restrict__ gd_part, const float* __restrict__ gbc,
                   const float* __restrict__ A_log, typename Elem<DT>::T* __restrict__ gB,
                   typename Elem<DT>::T* __restrict__ gC, float* __restrict__ gA_log, float* __restrict__ gD,
-                  int64_t N, int T, int Dn, int S, int nblk, int nga, int ngd) {
+                  int64_t N, int64_t parts, int T, int Dn, int S, int SP, int nblk, int nga, int ngd) {
   using E = Elem<DT>;
   __shared__ float red[16][64];
   const int bx = blockIdx.x;
@@ -411,7 +338,7 @@ ssm_scan_bwd_tail(const float* __restrict__ ga_part, const float* __restrict__ g
     float acc = 0.f;
     if (col < ncols) {
 #pragma unroll 8
-      for (int64_t n = rg; n < N; n += 16) acc += part[n * ncols + col];
+      for (int64_t n = rg; n < parts; n += 16) acc += part[n * ncols + col];
     }
     red[rg][c] = acc;
     __syncthreads();
@@ -477,6 +404,21 @@ static BwdWs bwd_ws(int64_t N, int64_t T, int64_t Dn, int64_t S) {
   return w;
 }
 
+// the tail launch: gA_log and gD reductions over `parts` partials and the sums of nblk gB / gC blocks
+template <int DT, int MODE>
+static int launch_tail(const float* ga, const float* gd, const float* gbc, const float* A_log, void* gB, void* gC,
+                       float* gA_log, float* gD, int64_t N, int64_t parts, int64_t T, int64_t Dn, int64_t S, int SP,
+                       int nblk, hipStream_t st) {
+  using TT = typename Elem<DT>::T;
+  const int nga = (int)((Dn * SP + 63) / 64), ngd = gD ? (int)((Dn + 63) / 64) : 0;
+  int64_t g = (N * T * S + 1023) / 1024;
+  g = g < 1 ? 1 : (g > 1024 ? 1024 : g);
+  hipLaunchKernelGGL((ssm_scan_bwd_tail<DT, MODE>), dim3((unsigned)(nga + ngd + g)), dim3(1024), 0, st, ga, gd, gbc,
+                     A_log, (TT*)gB, (TT*)gC, gA_log, gD, N, parts, (int)T, (int)Dn, (int)S, SP, nblk, nga, ngd);
+  HCLSM_LAUNCH_CHECK();
+  return 0;
+}
+
 template <int DT, int SP, int MODE>
 static int launch_bwd(const void* x, const void* dt, const float* A_log, const void* B, const void* C,
                       const float* Dskip, const void* gy, void* gx, void* gdt, float* gA_log, void* gB, void* gC,
@@ -498,15 +440,8 @@ static int launch_bwd(const void* x, const void* dt, const float* A_log, const v
                      (TT*)gdt, reinterpret_cast<float*>(ws + L.ck), gbc, reinterpret_cast<float*>(ws + L.ga),
                      reinterpret_cast<float*>(ws + L.gd), a);
   HCLSM_LAUNCH_CHECK();
-  // the tail: gA_log and gD reductions and the gB / gC block sums, one launch
-  const int nga = (int)((Dn * SP + 63) / 64), ngd = gD ? (int)((Dn + 63) / 64) : 0;
-  int64_t g = (N * T * S + 1023) / 1024;
-  g = g < 1 ? 1 : (g > 1024 ? 1024 : g);
-  hipLaunchKernelGGL((ssm_scan_bwd_tail<DT, SP, MODE>), dim3((unsigned)(nga + ngd + g)), dim3(1024), 0, st,
-                     reinterpret_cast<const float*>(ws + L.ga), reinterpret_cast<const float*>(ws + L.gd), gbc, A_log,
-                     (TT*)gB, (TT*)gC, gA_log, gD, N, (int)T, (int)Dn, (int)S, nblk_d, nga, ngd);
-  HCLSM_LAUNCH_CHECK();
-  return 0;
+  return launch_tail<DT, MODE>(reinterpret_cast<const float*>(ws + L.ga), reinterpret_cast<const float*>(ws + L.gd),
+                               gbc, A_log, gB, gC, gA_log, gD, N, N, T, Dn, S, SP, nblk_d, st);
 }
 
 }  // namespace hclsm
@@ -521,7 +456,8 @@ extern "C" int64_t hclsm_ssm_scan_bwd_workspace(int64_t batch, int64_t T, int64_
 static int scan_bwd_entry(const void* x, const void* dt, const float* A_log, const void* B, const void* C,
                           const float* Dskip, const void* gy, void* gx, void* gdt, float* gA_log, void* gB, void* gC,
                           float* gD, int64_t batch, int64_t T, int64_t d_inner, int64_t d_state, int dtype, int mode,
-                          void* workspace, int64_t workspace_bytes, bool have_ck, void* stream) {
+                          void* workspace, int64_t workspace_bytes, bool have_ck, void* stream,
+                          BwdGate gate = BwdGate()) {
   if (batch < 0 || T < 0 || d_inner < 0 || d_state < 1) return HCLSM_ERR_SHAPE;
   if (batch > 0x7fffffffLL || T > 0x7fffffffLL || d_inner > 0x7fffffffLL) return HCLSM_ERR_SHAPE;
   if (d_state > 128) return HCLSM_ERR_UNSUPPORTED;
@@ -544,6 +480,27 @@ static int scan_bwd_entry(const void* x, const void* dt, const float* A_log, con
   const BwdWs L = bwd_ws(batch, T, d_inner, d_state);
   if (workspace_bytes < (int64_t)L.total) return HCLSM_ERR_SHAPE;
   char* ws = reinterpret_cast<char*>(workspace);
+  if (!have_ck && bwd_group_ok(T, d_inner, d_state, dtype)) {
+    // wide states: their groups over the waves of a workgroup (its partials fit the regions of the layout above)
+    float* gbc = reinterpret_cast<float*>(ws + L.gbc);
+    float *ga = reinterpret_cast<float*>(ws + L.ga), *gd = reinterpret_cast<float*>(ws + L.gd);
+    int parts = 0;
+    const int rc = bwd_group(gate.gate ? BWD_BLOCK_GATE : mode, x, dt, A_log, B, C, Dskip, gy, gx, gdt, gate,
+                             reinterpret_cast<float*>(ws + L.ck), gbc, ga, gd, batch, T, d_inner, d_state, dtype, &parts,
+                             st);
+    if (rc) return rc;
+    const int nblk = (int)((d_inner + 63) / 64);
+#define HCLSM_TAIL(DT_, MODE_) \
+  return launch_tail<DT_, MODE_>(ga, gd, gbc, A_log, gB, gC, gA_log, gD, batch, parts, T, d_inner, d_state, (int)d_state, nblk, st)
+    if (dtype == HCLSM_F32) {
+      if (mode == HCLSM_SCAN_RAW) HCLSM_TAIL(HCLSM_F32, HCLSM_SCAN_RAW);
+      HCLSM_TAIL(HCLSM_F32, HCLSM_SCAN_MODEL);
+    }
+    if (mode == HCLSM_SCAN_RAW) HCLSM_TAIL(HCLSM_BF16, HCLSM_SCAN_RAW);
+    HCLSM_TAIL(HCLSM_BF16, HCLSM_SCAN_MODEL);
+#undef HCLSM_TAIL
+  }
+  if (gate.gate) return HCLSM_ERR_UNSUPPORTED;
 #define HCLSM_BWD(DT_, SP_)                                                                                  \
   if (sp_of(d_state) == SP_) {                                                                               \
     if (mode == HCLSM_SCAN_RAW)                                                                              \
