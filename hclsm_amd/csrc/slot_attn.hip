@@ -1152,7 +1152,7 @@ __global__ void __launch_bounds__(256)
 linear_lds_f32_kernel(const float* __restrict__ X, int64_t ldx, const float* __restrict__ W, int64_t ldw,
                       const float* __restrict__ bias, const float* __restrict__ resid, int64_t ldr,
                       typename MM<OT>::T* __restrict__ Y, int64_t ldy, float* __restrict__ Y2, int64_t ldy2,
-                      int64_t M, int64_t N, int64_t K, int relu, float clamp_v, LinExt ext) {
+                      int64_t M, int64_t N, int64_t K, int relu, float clamp_v, OutSplit os, LinExt ext) {
   __shared__ __align__(16) float As[64 * LF_LD];
   __shared__ __align__(16) float Bs[64 * LF_LD];
   const int64_t tiles_n = (N + 63) / 64;
@@ -1246,6 +1246,14 @@ linear_lds_f32_kernel(const float* __restrict__ X, int64_t ldx, const float* __r
     for (int ti = 0; ti < 2; ++ti) {
       const int64_t row = r0 + 16 * ti + li;
       if (row >= M || col >= N) continue;
+      if (os.yt != nullptr && col >= os.col) {   // transposed part (plain products): 16 rows of a column per line
+        const int64_t fr = row / os.frame_rows, rr = row - fr * os.frame_rows;
+        auto* yt = reinterpret_cast<typename MM<OT>::T*>(os.yt) + fr * os.bstride + (col - os.col) * os.ldyt + rr;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col + r < N) yt[r * os.ldyt] = MM<OT>::fromf(acc[ti][tj][r] + bv[r]);
+        continue;
+      }
       lin_epilogue4<HCLSM_F32, OT>(acc[ti][tj], bv, row, col, N, relu, clamp_v, resid, ldr, Y, ldy, Y2, ldy2, ext,
                                    vec);
     }
@@ -1322,7 +1330,20 @@ linear_quad_kernel(const typename MM<DT>::T* __restrict__ X, int64_t ldx, const 
   }
 }
 
-template <int DT, int OT, typename XT, bool LN>
+// fp32 contraction in 16-wide blocks (V4 kernels): lane group g loads k = 4g .. 4g+3 of a block as one float4 per
+// operand, and product j contracts the four k = 4g + j.  The scalar form loads one float per lane and product, so
+// every product waits on its own load round.  MI355X, fp32 forward of 32 frames x 196 tokens, 32 slots of 192, five
+// iterations (us per launch, scalar -> float4): linear layers 20.8 -> 9.2 (mean of three), GRU 30.0 -> 12.9, logits
+// 14.1 -> 8.0; with the update and k/v kernels below 1054 -> 335 per call.
+__device__ __forceinline__ f32x4 mfma_f32_k16(float4 a, float4 b, f32x4 c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+}
+
+// V4: fp32, K % 16 == 0, 16-byte rows (checked by the launcher).
+template <int DT, int OT, typename XT, bool LN, bool V4 = false>
 __global__ void __launch_bounds__(256)
 linear_kernel(const XT* __restrict__ X, int64_t ldx, const typename MM<DT>::T* __restrict__ W, int64_t ldw,
               const float* __restrict__ bias, const float* __restrict__ resid, int64_t ldr,
@@ -1330,7 +1351,8 @@ linear_kernel(const XT* __restrict__ X, int64_t ldx, const typename MM<DT>::T* _
               int64_t M, int64_t N, int64_t K, int relu, float clamp_v, const float* __restrict__ lnw,
               const float* __restrict__ lnb, float ln_eps, LinExt ext) {
   using A = MM<DT>;
-  constexpr int KPL = A::KPL;
+  static_assert(!V4 || (DT == HCLSM_F32 && !LN), "V4: fp32 without LayerNorm");
+  constexpr int KPL = V4 ? 4 : A::KPL;
   constexpr int BLK = 4 * KPL;
   __shared__ float red[4][2][2][4][64];   // [wave][ti][tj][r][lane]: 16 KB
   const int64_t tiles_n = (N + 31) / 32;
@@ -1357,6 +1379,22 @@ linear_kernel(const XT* __restrict__ X, int64_t ldx, const typename MM<DT>::T* _
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int nblk = (int)(K / BLK);
+  if constexpr (V4) {
+#pragma unroll 4
+    for (int s = wid; s < nblk; s += 4) {
+      const int64_t k0 = (int64_t)s * BLK;
+      float4 a[2], b[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        a[t] = *reinterpret_cast<const float4*>(pa[t] + k0);
+        b[t] = *reinterpret_cast<const float4*>(pb[t] + k0);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma_f32_k16(a[i], b[j], acc[i][j]);
+    }
+  } else
 #pragma unroll 2
   for (int s = wid; s < nblk; s += 4) {
     const int64_t k0 = (int64_t)s * BLK;
@@ -1659,7 +1697,8 @@ linear_kreg_kernel(const XT* __restrict__ X, int64_t ldx, const typename MM<DT>:
 // ---------------------------------------------------------------------------
 // GH: the hidden-side products come precomputed in gh ([M][3H] fp32, row stride ldgh, without b_hh); Hb and Whh
 // are not read.
-template <int DT, bool GH>
+// V4: fp32 with K and H multiples of 16 and 16-byte rows (mfma_f32_k16).
+template <int DT, bool GH, bool V4 = false>
 __global__ void __launch_bounds__(256)
 gru_kernel(const typename MM<DT>::T* __restrict__ X, int64_t ldx, const typename MM<DT>::T* __restrict__ Hb,
            int64_t ldhb, const float* __restrict__ Hf, int64_t ldh, const typename MM<DT>::T* __restrict__ Wih,
@@ -1667,9 +1706,28 @@ gru_kernel(const typename MM<DT>::T* __restrict__ X, int64_t ldx, const typename
            float* __restrict__ out, int64_t ldo, typename MM<DT>::T* __restrict__ out2, int64_t ldo2, int64_t M,
            int64_t H, int64_t Kx, const float* __restrict__ gh, int64_t ldgh) {
   using A = MM<DT>;
-  constexpr int KPL = A::KPL;
+  constexpr int KPL = V4 ? 4 : A::KPL;
   constexpr int BLK = 4 * KPL;
   constexpr int NQ = GH ? 3 : 6;         // products formed here
+  auto products = [&](const typename A::T* const* pa, const typename A::T* const* pw, int64_t k0, f32x4* c0, f32x4* c1) {
+    if constexpr (V4) {
+      const float4 a0 = *reinterpret_cast<const float4*>(pa[0] + k0), a1 = *reinterpret_cast<const float4*>(pa[1] + k0);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const float4 bq = *reinterpret_cast<const float4*>(pw[q] + k0);
+        c0[q] = mfma_f32_k16(a0, bq, c0[q]);
+        c1[q] = mfma_f32_k16(a1, bq, c1[q]);
+      }
+    } else {
+      const typename A::Op a0 = A::load(pa[0] + k0), a1 = A::load(pa[1] + k0);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const typename A::Op bq = A::load(pw[q] + k0);
+        c0[q] = A::mfma(a0, bq, c0[q]);
+        c1[q] = A::mfma(a1, bq, c1[q]);
+      }
+    }
+  };
   __shared__ float red[4][2][NQ][4][64];  // 48 KB (24 KB with GH)
   const int64_t tiles_n = (H + 15) / 16;
   const int64_t tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
@@ -1712,32 +1770,14 @@ gru_kernel(const typename MM<DT>::T* __restrict__ X, int64_t ldx, const typename
     const typename A::T* pw[3] = {Wih + colr * Kx + KPL * g, Wih + (H + colr) * Kx + KPL * g,
                                   Wih + (2 * H + colr) * Kx + KPL * g};
     const int nblk = (int)(Kx / BLK);
-    for (int s = wid; s < nblk; s += 4) {
-      const int64_t k0 = (int64_t)s * BLK;
-      const typename A::Op a0 = A::load(pa[0] + k0), a1 = A::load(pa[1] + k0);
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const typename A::Op bq = A::load(pw[q] + k0);
-        acc[0][q] = A::mfma(a0, bq, acc[0][q]);
-        acc[1][q] = A::mfma(a1, bq, acc[1][q]);
-      }
-    }
+    for (int s = wid; s < nblk; s += 4) products(pa, pw, (int64_t)s * BLK, acc[0], acc[1]);
   }
   if constexpr (!GH) {
     const typename A::T* pa[2] = {Hb + rows[0] * ldhb + KPL * g, Hb + rows[1] * ldhb + KPL * g};
     const typename A::T* pw[3] = {Whh + colr * H + KPL * g, Whh + (H + colr) * H + KPL * g,
                                   Whh + (2 * H + colr) * H + KPL * g};
     const int nblk = (int)(H / BLK);
-    for (int s = wid; s < nblk; s += 4) {
-      const int64_t k0 = (int64_t)s * BLK;
-      const typename A::Op a0 = A::load(pa[0] + k0), a1 = A::load(pa[1] + k0);
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const typename A::Op bq = A::load(pw[q] + k0);
-        acc[0][3 + q] = A::mfma(a0, bq, acc[0][3 + q]);
-        acc[1][3 + q] = A::mfma(a1, bq, acc[1][3 + q]);
-      }
-    }
+    for (int s = wid; s < nblk; s += 4) products(pa, pw, (int64_t)s * BLK, acc[0] + 3, acc[1] + 3);
   }
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -1785,13 +1825,14 @@ constexpr int CORE_MAX_NT = 8;  // up to 128 slots
 // Grid (frame, 16-token tile); the 4 waves split the D blocks, partial logits meet in LDS and
 // wave 0 finishes the softmax over slots.
 // NWL waves split the contraction (8 for fp32 on a grid that fills few CUs: half the blocks per wave).
-template <int DT, int AT, int NWL = 4>
+// V4: fp32 with D % 16 == 0 and 16-byte rows (mfma_f32_k16).
+template <int DT, int AT, int NWL = 4, bool V4 = false>
 __global__ void __launch_bounds__(64 * NWL)
 core_logits_kernel(const typename MM<DT>::T* __restrict__ q, const typename MM<DT>::T* __restrict__ k,
                    typename MM<DT>::T* __restrict__ P, int64_t Mp, float* __restrict__ part,
                    typename MM<AT>::T* __restrict__ attn_out, CoreArgs a) {
   using A = MM<DT>;
-  constexpr int KPL = A::KPL;
+  constexpr int KPL = V4 ? 4 : A::KPL;
   constexpr int BLK = 4 * KPL;
   __shared__ float red[NWL][CORE_MAX_NT][4][64];   // 32 KB (64 KB with eight waves)
   const int64_t b = blockIdx.x;
@@ -1811,6 +1852,16 @@ core_logits_kernel(const typename MM<DT>::T* __restrict__ q, const typename MM<D
     n = n < a.N ? n : a.N - 1;
     qrow[nt] = q + b * a.qb + (int64_t)n * a.ldq + KPL * g;
   }
+  if constexpr (V4) {
+#pragma unroll 3
+    for (int s = wid; s < nblk; s += NWL) {
+      const float4 kb_ = *reinterpret_cast<const float4*>(kp + (int64_t)s * BLK);
+#pragma unroll
+      for (int nt = 0; nt < CORE_MAX_NT; ++nt)
+        if (nt < a.NT)
+          acc[nt] = mfma_f32_k16(*reinterpret_cast<const float4*>(qrow[nt] + (int64_t)s * BLK), kb_, acc[nt]);
+    }
+  } else
 #pragma unroll 2
   for (int s = wid; s < nblk; s += NWL) {
     const typename A::Op kb_ = A::load(kp + (int64_t)s * BLK);
@@ -1924,7 +1975,7 @@ core_update_t_kernel(const typename MM<DT>::T* __restrict__ P, int64_t Mp, const
   float cs = 0.f;
 #pragma unroll 2
   for (int m0 = 0; m0 < (int)Mp; m0 += 32) {
-    if constexpr (KPL == 8) {
+    {
       typename A::Op bv = A::load(pv + m0 + 8 * g);
       if (m0 + 32 > a.M) {   // tokens past M: v rows are not initialised, zero them
         TT e[8];
@@ -1943,16 +1994,6 @@ core_update_t_kernel(const typename MM<DT>::T* __restrict__ P, int64_t Mp, const
 #pragma unroll
       for (int nt = 0; nt < CORE_MAX_NT; ++nt)
         if (nt < a.NT) acc[nt] = A::mfma(A::load(prow[nt] + m0 + 8 * g), bv, acc[nt]);
-    } else {
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const int mm = m0 + 4 * s + g;
-        float bv = mm < a.M ? pv[mm] : 0.f;
-        if (renorm) cs += bv;
-#pragma unroll
-        for (int nt = 0; nt < CORE_MAX_NT; ++nt)
-          if (nt < a.NT) acc[nt] = A::mfma(prow[nt][mm], bv, acc[nt]);
-      }
     }
   }
   cs = rows4_sum(cs);
@@ -1966,6 +2007,71 @@ core_update_t_kernel(const typename MM<DT>::T* __restrict__ P, int64_t Mp, const
       const int n = nt * 16 + 4 * g + r;
       if (n < a.N) out[b * a.ob + (int64_t)n * a.ldo + d] = A::fromf((acc[nt][r] + epsv) * rinv_s[n]);
     }
+  }
+}
+
+// The same for fp32: grid (frame, 16-column tile), the 4 waves splitting the tokens in 16-wide blocks (mfma_f32_k16)
+// and meeting in LDS.  (One wave per 16 columns over all tokens, a float per lane and product, left 96 workgroups
+// waiting on 56 dependent load rounds: 68.3 us against 7.3 at 32 frames x 196 tokens x 192, 32 slots.)
+__global__ void __launch_bounds__(256)
+core_update_t_f32_kernel(const float* __restrict__ P, int64_t Mp, const float* __restrict__ part,
+                         const float* __restrict__ vt, float* __restrict__ out, CoreArgs a) {
+  __shared__ float red[4][CORE_MAX_NT][4][64];
+  __shared__ float csum[4][16];
+  __shared__ float rinv_s[CORE_MAX_NT * 16];
+  const int64_t b = blockIdx.x;
+  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63, g = lane >> 4, li = lane & 15;
+  const int d = blockIdx.y * 16 + li;
+  const int dc = d < a.D ? d : a.D - 1;
+  const bool renorm = a.renorm_eps >= 0.f;
+  if (tid < a.NT * 16) {
+    float s = 1.f;
+    if (renorm && tid < a.N) {
+      float t = 0.f;
+      for (int j = 0; j < a.MT; ++j) t += part[(b * a.MT + j) * a.N + tid];
+      s = 1.f / (t + (float)a.M * a.renorm_eps);
+    }
+    rinv_s[tid] = s;
+  }
+  const float* pv = vt + b * a.vb + (int64_t)dc * Mp + 4 * g;
+  const float* prow[CORE_MAX_NT];
+#pragma unroll
+  for (int nt = 0; nt < CORE_MAX_NT; ++nt) {
+    int n = nt * 16 + li;
+    n = n < a.N ? n : a.N - 1;
+    prow[nt] = P + (b * a.N + n) * Mp + 4 * g;
+  }
+  f32x4 acc[CORE_MAX_NT];
+#pragma unroll
+  for (int nt = 0; nt < CORE_MAX_NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float cs = 0.f;
+#pragma unroll 4
+  for (int m0 = 16 * wid; m0 < (int)Mp; m0 += 64) {
+    float4 bv = *reinterpret_cast<const float4*>(pv + m0);
+    const int m = m0 + 4 * g;              // tokens past M: v rows are not initialised, zero them (P is zero there)
+    bv.x = m < a.M ? bv.x : 0.f;
+    bv.y = m + 1 < a.M ? bv.y : 0.f;
+    bv.z = m + 2 < a.M ? bv.z : 0.f;
+    bv.w = m + 3 < a.M ? bv.w : 0.f;
+    if (renorm) cs += (bv.x + bv.y) + (bv.z + bv.w);
+#pragma unroll
+    for (int nt = 0; nt < CORE_MAX_NT; ++nt)
+      if (nt < a.NT) acc[nt] = mfma_f32_k16(*reinterpret_cast<const float4*>(prow[nt] + m0), bv, acc[nt]);
+  }
+  cs = rows4_sum(cs);
+  if (g == 0) csum[wid][li] = cs;
+#pragma unroll
+  for (int nt = 0; nt < CORE_MAX_NT; ++nt)
+    if (nt < a.NT)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wid][nt][r][lane] = acc[nt][r];
+  __syncthreads();
+  if (d >= a.D) return;
+  const float epsv = renorm ? a.renorm_eps * (csum[0][li] + csum[1][li] + csum[2][li] + csum[3][li]) : 0.f;
+  for (int u = wid; u < 4 * a.NT; u += 4) {
+    const int nt = u >> 2, r = u & 3, n = nt * 16 + 4 * g + r;
+    const float s = red[0][nt][r][lane] + red[1][nt][r][lane] + red[2][nt][r][lane] + red[3][nt][r][lane];
+    if (n < a.N) out[b * a.ob + (int64_t)n * a.ldo + d] = (s + epsv) * rinv_s[n];
   }
 }
 
@@ -2493,19 +2599,32 @@ static int launch_core(const void* q, int64_t ldq, int64_t qbs, const void* k, i
   float* part = reinterpret_cast<float*>(reinterpret_cast<char*>(ws) + poff);
   dim3 g1((unsigned)B, (unsigned)(Mp / 16));
   dim3 g2((unsigned)B, (unsigned)((D + CORE_DB - 1) / CORE_DB));
+  if (dtype == HCLSM_F32 && (attn == nullptr || attn_dtype == HCLSM_F32)) {
+    // rows of q and k as float4 (D % 16 == 0: check_core); eight waves a tile on a grid that fills few CUs
+    const bool v4 = al16(q) && al16(k) && ldq % 4 == 0 && ldk % 4 == 0 && qbs % 4 == 0 && kbs % 4 == 0 && D % 16 == 0;
+    const bool few = B * (Mp / 16) < 128;
+    const auto kern = v4 ? (few ? core_logits_kernel<HCLSM_F32, HCLSM_F32, 8, true> : core_logits_kernel<HCLSM_F32, HCLSM_F32, 4, true>)
+                         : (few ? core_logits_kernel<HCLSM_F32, HCLSM_F32, 8> : core_logits_kernel<HCLSM_F32, HCLSM_F32>);
+    hipLaunchKernelGGL(kern, g1, dim3(few ? 512 : 256), 0, st, (const float*)q, (const float*)k, (float*)ws, Mp, part,
+                       (float*)attn, a);
+    HCLSM_LAUNCH_CHECK();
+    if (v_transposed)
+      hipLaunchKernelGGL(core_update_t_f32_kernel, dim3((unsigned)B, (unsigned)((D + 15) / 16)), dim3(256), 0, st,
+                         (const float*)ws, Mp, part, (const float*)v, (float*)out, a);
+    else
+      launch_update_plain<HCLSM_F32>((const float*)ws, Mp, part, (const float*)v, (float*)out, a, B, D, g2, st);
+    HCLSM_LAUNCH_CHECK();
+    return 0;
+  }
 #define HCLSM_CORE(D_, A_)                                                                                   \
   if (dtype == D_ && (attn == nullptr ? A_ == D_ : attn_dtype == A_)) {                                      \
-    if (D_ == HCLSM_F32 && B * (Mp / 16) < 128)                                                              \
-      hipLaunchKernelGGL((core_logits_kernel<D_, A_, 8>), g1, dim3(512), 0, st, (const MM<D_>::T*)q,         \
-                         (const MM<D_>::T*)k, (MM<D_>::T*)ws, Mp, part, (MM<A_>::T*)attn, a);                \
-    else                                                                                                     \
-      hipLaunchKernelGGL((core_logits_kernel<D_, A_>), g1, dim3(256), 0, st, (const MM<D_>::T*)q,           \
-                         (const MM<D_>::T*)k, (MM<D_>::T*)ws, Mp, part, (MM<A_>::T*)attn, a);                \
+    hipLaunchKernelGGL((core_logits_kernel<D_, A_>), g1, dim3(256), 0, st, (const MM<D_>::T*)q,             \
+                       (const MM<D_>::T*)k, (MM<D_>::T*)ws, Mp, part, (MM<A_>::T*)attn, a);                  \
     HCLSM_LAUNCH_CHECK();                                                                                    \
     if (v_transposed)                                                                                        \
       hipLaunchKernelGGL((core_update_t_kernel<D_>), g2, dim3(256), 0, st, (const MM<D_>::T*)ws, Mp, part,   \
                          (const MM<D_>::T*)v, (MM<D_>::T*)out, a);                                           \
-    else                                                                                                     \
+    else                                                                                                   \
       launch_update_plain<D_>((const MM<D_>::T*)ws, Mp, part, (const MM<D_>::T*)v, (MM<D_>::T*)out, a, B, D, g2, st); \
     HCLSM_LAUNCH_CHECK();                                                                                    \
     return 0;                                                                                                \
@@ -2514,7 +2633,6 @@ static int launch_core(const void* q, int64_t ldq, int64_t qbs, const void* k, i
   HCLSM_CORE(HCLSM_BF16, HCLSM_F32)
   HCLSM_CORE(HCLSM_F16, HCLSM_F16)
   HCLSM_CORE(HCLSM_F16, HCLSM_F32)
-  HCLSM_CORE(HCLSM_F32, HCLSM_F32)
 #undef HCLSM_CORE
   return HCLSM_ERR_DTYPE;
 }
@@ -2626,10 +2744,13 @@ static void launch_linear_quad(const void* x, int64_t ldx, const void* w, int64_
                            ldx, (const typename MM<DT>::T*)w, ldw, bias, resid, ldr, (typename MM<OT>::T*)y, ldy,
                            (typename MM<DT>::T*)y2, ldy2, M, N, K, relu, clamp, os, ext);
     } else if constexpr (direct) {
-      if (os.yt == nullptr && al16(x) && al16(w) && ldx % 4 == 0 && ldw % 4 == 0)
+      // (a transposed part starts on a column multiple of 4 and takes the products as they are; k/v projection of
+      // 6272 x 384 x 384: 134.8 us with direct scalar loads, 30.1 through LDS)
+      const bool split_ok = os.yt == nullptr || (os.col % 4 == 0 && !relu && !resid && !y2 && clamp <= 0.f && K % 4 == 0);
+      if (split_ok && al16(x) && al16(w) && ldx % 4 == 0 && ldw % 4 == 0)
         hipLaunchKernelGGL((linear_lds_f32_kernel<OT>), dim3(grid), dim3(256), 0, st, (const float*)x, ldx,
                            (const float*)w, ldw, bias, resid, ldr, (typename MM<OT>::T*)y, ldy, (float*)y2, ldy2, M,
-                           N, K, relu, clamp, ext);
+                           N, K, relu, clamp, os, ext);
       else
         hipLaunchKernelGGL((linear_quad_kernel<DT, OT>), dim3(grid), dim3(256), 0, st, (const typename MM<DT>::T*)x,
                            ldx, (const typename MM<DT>::T*)w, ldw, bias, resid, ldr, (typename MM<OT>::T*)y, ldy,
@@ -2692,6 +2813,14 @@ static void launch_linear_t(bool ln, const void* x, int64_t ldx, const void* w, 
     }
   }
   const unsigned grid = (unsigned)tiles32;
+  if constexpr (DT == HCLSM_F32) {
+    if (!ln && K % 16 == 0 && al16(x) && al16(w) && ldx % 4 == 0 && ldw % 4 == 0) {
+      hipLaunchKernelGGL((linear_kernel<DT, OT, XT, false, true>), dim3(grid), dim3(256), 0, st, (const XT*)x, ldx,
+                         (const typename MM<DT>::T*)w, ldw, bias, resid, ldr, (typename MM<OT>::T*)y, ldy,
+                         (typename MM<DT>::T*)y2, ldy2, M, N, K, relu, clamp, lnw, lnb, eps, ext);
+      return;
+    }
+  }
   if (ln)
     hipLaunchKernelGGL((linear_kernel<DT, OT, XT, true>), dim3(grid), dim3(256), 0, st, (const XT*)x, ldx,
                        (const typename MM<DT>::T*)w, ldw, bias, resid, ldr, (typename MM<OT>::T*)y, ldy,
@@ -2907,6 +3036,14 @@ static int gru_impl(const void* x, int64_t ldx, const void* hb, int64_t ldhb, co
   if (kpl == 8 && (!al16(x) || !al16(w_ih) || ldx % 8)) return HCLSM_ERR_UNSUPPORTED;
   if (kpl == 8 && !gh && (!al16(hb) || !al16(w_hh) || ldhb % 8)) return HCLSM_ERR_UNSUPPORTED;
   const unsigned grid = (unsigned)(((M + 31) / 32) * ((H + 15) / 16));
+  if (dtype == HCLSM_F32 && !gh && Kx % 16 == 0 && H % 16 == 0 && al16(x) && al16(hb) && al16(w_ih) && al16(w_hh) &&
+      ldx % 4 == 0 && ldhb % 4 == 0) {
+    hipLaunchKernelGGL((gru_kernel<HCLSM_F32, false, true>), dim3(grid), dim3(256), 0, st, (const float*)x, ldx,
+                       (const float*)hb, ldhb, h, ldh, (const float*)w_ih, (const float*)w_hh, b_ih, b_hh, out, ldo,
+                       (float*)out2, ldo2, M, H, Kx, gh, ldgh);
+    HCLSM_LAUNCH_CHECK();
+    return 0;
+  }
 #define HCLSM_GRU(D)                                                                                        \
   if (dtype == D) {                                                                                         \
     if (gh)                                                                                                 \
