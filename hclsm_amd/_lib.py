@@ -38,6 +38,10 @@ _SIGNATURES: dict[str, list] = {
     "hclsm_ssm_scan_fwd_ckpt": [_c_void_p] * 8 + [_i64] * 4 + [_int, _int, _c_void_p, _i64, _c_void_p],
     "hclsm_ssm_block_scan_fwd_ckpt": [_c_void_p] * 9 + [_i64] * 4 + [_int, _c_void_p, _i64, _c_void_p],
     "hclsm_ssm_scan_bwd_ckpt": [_c_void_p] * 13 + [_i64] * 4 + [_int, _int, _c_void_p, _i64, _c_void_p],
+    "hclsm_ssm_block_save": [_i64] * 5 + [_int],
+    "hclsm_ssm_block_scratch": [_i64] * 5,
+    "hclsm_ssm_block_forward": [_c_void_p] * 3 + [_i64] * 5 + [_int, _c_void_p, _i64, _c_void_p],
+    "hclsm_ssm_block_backward": [_c_void_p] * 5 + [_i64] * 5 + [_c_void_p, _i64, _c_void_p, _i64, _c_void_p],
     "hclsm_event_index": [_c_void_p, _int, _i64, _i64, _int] + [_c_void_p] * 6 + [_c_void_p],
     "hclsm_event_gather": [_c_void_p, _c_void_p, _i64, _i64, _i64, _i64] + [_c_void_p] * 3 + [_c_void_p],
     "hclsm_event_gather_packed": [_c_void_p, _c_void_p, _i64, _i64, _i64, _i64] + [_c_void_p] * 3 + [_c_void_p],
@@ -88,7 +92,8 @@ _SIGNATURES: dict[str, list] = {
     "hclsm_issue_probe": [_int, _i64, _int, _c_void_p, _c_void_p],
 }
 _RESTYPES = {"hclsm_strerror": ctypes.c_char_p, "hclsm_slot_attn_core_workspace": ctypes.c_int64,
-             "hclsm_ssm_scan_bwd_workspace": ctypes.c_int64,
+             "hclsm_ssm_scan_bwd_workspace": ctypes.c_int64, "hclsm_ssm_block_save": ctypes.c_int64,
+             "hclsm_ssm_block_scratch": ctypes.c_int64,
              "hclsm_slot_attention_workspace": ctypes.c_int64, "hclsm_slot_attention_k_offset": ctypes.c_int64,
              "hclsm_slot_attention_kq_offset": ctypes.c_int64, "hclsm_level1_forward_workspace": ctypes.c_int64,
              "hclsm_relation_graph_workspace": ctypes.c_int64, "hclsm_slot_track_cost_workspace": ctypes.c_int64,

@@ -522,6 +522,14 @@ static int scan_bwd_entry(const void* x, const void* dt, const float* A_log, con
   return HCLSM_ERR_UNSUPPORTED;
 }
 
+int hclsm::scan_bwd_block(const void* z, const void* dt_in, const float* A_log, const void* B, const void* C,
+                          const void* gy, void* gz, void* gdt, float* gA_log, void* gB, void* gC, int64_t batch, int64_t T,
+                          int64_t d_inner, int64_t d_state, int dtype, BwdGate gate, void* ws, int64_t ws_bytes,
+                          bool have_ck, hipStream_t st) {
+  return scan_bwd_entry(z, dt_in, A_log, B, C, nullptr, gy, gz, gdt, gA_log, gB, gC, nullptr, batch, T, d_inner, d_state,
+                        dtype, HCLSM_SCAN_BLOCK, ws, ws_bytes, have_ck, (void*)st, gate);
+}
+
 extern "C" int hclsm_ssm_scan_bwd(const void* x, const void* dt, const float* A_log, const void* B, const void* C,
                                   const float* Dskip, const void* gy, void* gx, void* gdt, float* gA_log, void* gB,
                                   void* gC, float* gD, int64_t batch, int64_t T, int64_t d_inner, int64_t d_state,

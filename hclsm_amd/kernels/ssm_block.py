@@ -1,0 +1,127 @@
+"""A whole SimplifiedSSMBlock (hclsm/dynamics/level0_ssm.py:30-107) under a bf16 autocast on MI355X
+(libhclsm_amd.so: hclsm_ssm_block_forward / hclsm_ssm_block_backward): one library call each way, with the
+roundings of the module's ops (bf16 operands and intermediates, fp32 residual stream, parameters and gradients).
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import torch
+import torch.nn as nn
+
+from hclsm_amd import _lib
+
+_NAMES = ("ln_w", "ln_b", "w_in", "w_gate", "w_dt", "b_dt", "w_b", "w_c", "a_log", "w_out")
+
+
+class _Ptrs(ctypes.Structure):
+    """Mirror of the C structs HclsmBlockParams / HclsmBlockGrads (the same ten pointers)."""
+    _fields_ = [(n, ctypes.c_void_p) for n in _NAMES]
+
+
+def _ptrs(tensors) -> _Ptrs:
+    return _Ptrs(*(t.data_ptr() for t in tensors))
+
+
+def _plain_linear(m, bias: bool) -> bool:
+    return type(m) is nn.Linear and (m.bias is not None) == bias and _no_hooks(m)
+
+
+def _no_hooks(m) -> bool:
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+
+
+def block_params(m, x):
+    """The block's parameters in _NAMES order where the fused block computes what the module's ops would (bf16 autocast,
+    fp32 input and parameters, plain submodules nobody hooks into, no tracing or function transform), else None."""
+    if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.numel() > 0 and type(x) in (torch.Tensor, nn.Parameter)):
+        return None
+    if not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") != torch.bfloat16:
+        return None
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._are_functorch_transforms_active():
+        return None
+    if torch.autograd.forward_ad._current_level >= 0:
+        return None
+    mm = nn.modules.module
+    if mm._global_forward_hooks or mm._global_forward_pre_hooks or mm._global_backward_hooks or mm._global_backward_pre_hooks:
+        return None
+    norm = m.norm
+    if type(norm) is not nn.LayerNorm or norm.eps != 1e-5 or norm.bias is None or not _no_hooks(norm):
+        return None
+    if not (all(_plain_linear(p, False) for p in (m.in_proj, m.gate_proj, m.B_proj, m.C_proj, m.out_proj))
+            and _plain_linear(m.dt_proj, True)):
+        return None
+    ps = (norm.weight, norm.bias, m.in_proj.weight, m.gate_proj.weight, m.dt_proj.weight, m.dt_proj.bias,
+          m.B_proj.weight, m.C_proj.weight, m.A_log, m.out_proj.weight)
+    dev = x.device
+    if any(type(p) not in (nn.Parameter, torch.Tensor) or p.dtype != torch.float32 or p.device != dev or
+           not p.is_contiguous() for p in ps):
+        return None
+    d, di, S = x.shape[2], m.A_log.shape[0], m.A_log.shape[1]
+    want = ((d,), (d,), (di, d), (di, d), (di, di), (di,), (S, di), (S, di), (di, S), (d, di))
+    if any(tuple(p.shape) != s for p, s in zip(ps, want)):
+        return None
+    return ps
+
+
+def _save_buffer(x, ps, train: bool):
+    N, T, d = x.shape
+    nb = int(_lib.lib().hclsm_ssm_block_save(N, T, d, ps[8].shape[0], ps[8].shape[1], int(train)))
+    return None if nb < 0 else torch.empty(nb, dtype=torch.uint8, device=x.device)
+
+
+def _forward(x, ps, save, train: bool):
+    N, T, d = x.shape
+    out = torch.empty_like(x)
+    st = _ptrs(ps)
+    return out, _lib.lib().hclsm_ssm_block_forward(
+        ctypes.byref(st), x.data_ptr(), out.data_ptr(), N, T, d, ps[8].shape[0], ps[8].shape[1], int(train),
+        save.data_ptr(), save.numel(), _lib.stream_of(x))
+
+
+class _Block(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, save, *ps):
+        out, rc = _forward(x, ps, save, True)
+        _lib.check(rc, "hclsm_ssm_block_forward")
+        ctx.save_for_backward(x, save, *ps)
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, g):
+        x, save, *ps = ctx.saved_tensors
+        N, T, d = x.shape
+        di, S = ps[8].shape
+        g = g.to(torch.float32).contiguous()
+        L = _lib.lib()
+        scratch = torch.empty(int(L.hclsm_ssm_block_scratch(N, T, d, di, S)), dtype=torch.uint8, device=x.device)
+        gx = torch.empty_like(x)
+        grads = [torch.empty_like(p) for p in ps]
+        st, sg = _ptrs(ps), _ptrs(grads)
+        rc = L.hclsm_ssm_block_backward(ctypes.byref(st), x.data_ptr(), g.data_ptr(), gx.data_ptr(), ctypes.byref(sg), N, T,
+                                        d, di, S, save.data_ptr(), save.numel(), scratch.data_ptr(), scratch.numel(),
+                                        _lib.stream_of(x))
+        _lib.check(rc, "hclsm_ssm_block_backward")
+        need = ctx.needs_input_grad
+        return (gx if need[0] else None, None, *(v if n else None for v, n in zip(grads, need[2:])))
+
+
+def ssm_block(m, x):
+    """The block's output, or None where this path does not apply (the caller runs the module's ops)."""
+    ps = block_params(m, x)
+    if ps is None:
+        return None
+    xc = x.contiguous()
+    train = torch.is_grad_enabled() and (xc.requires_grad or any(p.requires_grad for p in ps))
+    save = _save_buffer(xc, ps, train)
+    if save is None or (xc.data_ptr() | ps[0].data_ptr() | ps[1].data_ptr() | ps[8].data_ptr()) & 15:
+        return None
+    if train:
+        return _Block.apply(xc, save, *ps)
+    out, rc = _forward(xc, ps, save, False)
+    if rc == _lib.ERR_UNSUPPORTED:
+        return None
+    _lib.check(rc, "hclsm_ssm_block_forward")
+    return out

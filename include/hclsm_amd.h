@@ -150,6 +150,40 @@ int hclsm_ssm_scan_bwd_ckpt(const void* x, const void* dt, const float* A_log, c
                             int dtype, int mode, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * One SimplifiedSSMBlock in bf16 operands (what a bf16 autocast computes): fp32 input x [batch, T, d_model], output and
+ * parameters; forward and backward in one call each.
+ *   out = x + (silu(gate) * scan(z, clamp(softplus(dt), 1e-3, 1), a_log, B, C)) w_out^T with u = LayerNorm(x),
+ *   z = u w_in^T, gate = u w_gate^T, dt = z w_dt^T + b_dt, B = z w_b^T, C = z w_c^T (eps 1e-5).
+ *   save:    hclsm_ssm_block_save bytes (256-byte aligned): intermediates; with train != 0 also what the backward reads.
+ *   scratch: hclsm_ssm_block_scratch bytes (256-byte aligned), backward only.
+ *   The backward takes the gradient g of out (fp32) and writes gx (x's, the residual included) and every parameter's
+ *   gradient (fp32, overwritten).  save must hold what a forward with train != 0 left for the same inputs.
+ * Limits: d_model, d_inner and d_state multiples of 8, d_model <= 1024, d_inner <= 4096, d_state 16 or 24 .. 128 (64 at
+ *   most where not a multiple of 16), batch * T <= 2^24, batch * T * d_inner < 2^30; HCLSM_ERR_UNSUPPORTED elsewhere.
+ * Replaces: SimplifiedSSMBlock.forward (hclsm/dynamics/level0_ssm.py:58-107) and its autograd under bf16 autocast.
+ */
+typedef struct HclsmBlockParams {
+  const float *ln_w, *ln_b;       /* [d_model] */
+  const float *w_in, *w_gate;     /* [d_inner, d_model] */
+  const float *w_dt, *b_dt;       /* [d_inner, d_inner], [d_inner] */
+  const float *w_b, *w_c;         /* [d_state, d_inner] */
+  const float *a_log;             /* [d_inner, d_state] */
+  const float *w_out;             /* [d_model, d_inner] */
+} HclsmBlockParams;
+typedef struct HclsmBlockGrads {
+  float *ln_w, *ln_b, *w_in, *w_gate, *w_dt, *b_dt, *w_b, *w_c, *a_log, *w_out;
+} HclsmBlockGrads;
+int64_t hclsm_ssm_block_save(int64_t batch, int64_t T, int64_t d_model, int64_t d_inner, int64_t d_state, int train);
+int64_t hclsm_ssm_block_scratch(int64_t batch, int64_t T, int64_t d_model, int64_t d_inner, int64_t d_state);
+int hclsm_ssm_block_forward(const HclsmBlockParams* params, const float* x, float* out, int64_t batch, int64_t T,
+                            int64_t d_model, int64_t d_inner, int64_t d_state, int train, void* save, int64_t save_bytes,
+                            void* stream);
+int hclsm_ssm_block_backward(const HclsmBlockParams* params, const float* x, const float* g, float* gx,
+                             const HclsmBlockGrads* grads, int64_t batch, int64_t T, int64_t d_model, int64_t d_inner,
+                             int64_t d_state, const void* save, int64_t save_bytes, void* scratch, int64_t scratch_bytes,
+                             void* stream);
+
+/*
  * Event index of a [B, T] mask, built on the device with no host synchronisation.
  *   counts  [B]      int32  events per row
  *   offsets [B+1]    int32  exclusive prefix sum of counts; offsets[B] = total
