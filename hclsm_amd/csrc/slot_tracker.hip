@@ -12,7 +12,8 @@
 // perm, alive permuted with them) against frame t.  Row i of that cost matrix is row perm_{t-1}[i] of the
 // cost between the unpermuted frames t-1 and t, penalties included.  So the pair MLP runs once, in one
 // launch, over every (t-1, t) frame pair of every clip; only the Sinkhorn matching is sequential in t: one
-// workgroup per clip loops over the frames with the previous perm and alive row in LDS.  The tracked slots
+// workgroup per clip loops over the frames with the previous perm and alive row in LDS, taking a frame pair's
+// match from the workgroups that match the pairs beside it where the order of the rows cannot matter.  The tracked slots
 // are gathered afterwards in one parallel pass.  The GRU hidden state (slot_tracker.py:137-158) does not
 // feed back into the matching; when it is wanted it is carried in a second loop, one GEMM and one gate
 // launch per frame, with the input-side GEMM done once for all frames.
@@ -323,15 +324,16 @@ track_cost_res_kernel(TrackCostArgs a) {
 }
 
 // y[r, k] = clamp(x[r, k], -50, 50) (NaN passes through, as torch.clamp); VW = 4: float4 units (n a multiple of
-// 4, x and y 16-byte aligned)
+// 4, x and y 16-byte aligned).  z (nullable): nz <= n / VW words to clear in the same launch
 __device__ __forceinline__ float trk_clamp1(float v) {
   return v < -TRK_SLOT_CLAMP ? -TRK_SLOT_CLAMP : (v > TRK_SLOT_CLAMP ? TRK_SLOT_CLAMP : v);
 }
 template <int VW>
 __global__ void __launch_bounds__(256)
-trk_clamp_kernel(const float* __restrict__ x, float* __restrict__ y, int64_t n) {
+trk_clamp_kernel(const float* __restrict__ x, float* __restrict__ y, int64_t n, int* __restrict__ z, int64_t nz) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n / VW) return;
+  if (z && e < nz) z[e] = 0;
   if constexpr (VW == 4) {
     float4 v = reinterpret_cast<const float4*>(x)[e];
     v.x = trk_clamp1(v.x); v.y = trk_clamp1(v.y); v.z = trk_clamp1(v.z); v.w = trk_clamp1(v.w);
@@ -488,23 +490,116 @@ track_match_kernel(const float* __restrict__ cost, const float* __restrict__ ali
   }
 }
 
-// The matching half of the tracking loop (model.py:233-252) for one clip per workgroup.  C: cost between
+// Matching of one frame pair ahead of the loop.  Step t of the tracking loop matches the rows of the (t-1, t) cost block
+// taken in tracked order.  Where those rows are the block's own rows in another order, the normalisation gives the same
+// matrix in that order (a row keeps its column order, so only the rounding of the column sums can differ), and row i's
+// match is sig[perm[i]] with sig the match of the block as it stands: every pair of every clip at once instead of one
+// after another.  Two things are needed:
+//  - the order is one of all rows, which the loop checks.  Dead slots repeat (they are matched to the lowest dead slot),
+//    but a row whose costs all sit at the clamp ("flat": a dead slot) equals every other flat row, so it is enough that
+//    every other row occurs once;
+//  - no decision is close: sig is written only if in every row the best entry is at least TRK_MARGIN (in log units)
+//    above the best one of another column (columns that are flat throughout are equal to the bit and count as one; the
+//    lowest wins in either order) and not near the 0.3 threshold, and the rows that are not flat take distinct columns.
+//    The rounding is 1e-7 of these values.
+// It gives up after TRK_EARLY rounds if the decisions clash already (untrained weights).
+// The loop is a serial chain: 20 normalisations of 0.55 us in each step, on one compute unit per clip, 724 us for 32
+// clips of 64 frames and 32 slots.  With the pairs ahead 80 us (steps 1 .. 3 by the loop, 0.8 us for each step after).
+// sig is read while it is written: each word is stored and loaded by itself at device scope, is 0 before this launch
+// and carries TRK_READY, so the loop needs no order between words and never waits.
+constexpr float TRK_MARGIN = 0.1f;
+constexpr int TRK_EARLY = 5;
+constexpr int TRK_READY = 1 << 30, TRK_FLAT = 1 << 29, TRK_CONF = 1 << 28, TRK_IDX = 0xffff;
+constexpr int TRK_AHEAD = 3;     // first frame matched ahead: by then the loop has run the steps before it
+
+// cf: the pair's cost block; sg: its N words; sL [NC][P], s_fc and s_cnt [NC] in LDS
+template <int CPL>
+__device__ __forceinline__ void track_pair(const float* __restrict__ cf, int* __restrict__ sg, float* sL, int* s_fc,
+                                           int* s_cnt, int line, int cg, int N, int n_iters, float inv_t) {
+  constexpr int P = SkTile<CPL>::P;
+  const float flat_v = la_of(TRK_COST_CLAMP, inv_t);
+  float v[CPL];
+  int fr = 1;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+    const int j = cg * CPL + c;
+    const bool in = line < N && j < N;
+    v[c] = in ? la_of(cf[(size_t)line * N + j], inv_t) : -INFINITY;
+    if (in && v[c] != flat_v) fr = 0;
+    sL[line * P + j] = v[c];
+  }
+  fr &= dpp_i<0xb1>(fr);
+  fr &= dpp_i<0x4e>(fr);
+  fr &= dpp_i<0x141>(fr);                   // row `line` is flat
+  __syncthreads();
+  int fc = 1;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c)
+    if (line < N && cg * CPL + c < N && sL[(cg * CPL + c) * P + line] != flat_v) fc = 0;
+  fc &= dpp_i<0xb1>(fc);
+  fc &= dpp_i<0x4e>(fc);
+  fc &= dpp_i<0x141>(fc);
+  if (cg == 0) s_fc[line] = fc;
+  float bv = 0.f;
+  int bi = 0;
+  for (int done = 0; done < n_iters;) {
+    const int some = n_iters - done > TRK_EARLY && done == 0 ? TRK_EARLY : n_iters - done;
+    if (cg == 0) s_cnt[line] = 0;
+    sinkhorn_lds<CPL>(sL, some, line, cg);   // ends on a barrier
+    done += some;
+    argmax_row<CPL>(sL, N, line, cg, bv, bi);
+    // the best entry outside the chosen column's class
+    const int bflat = s_fc[bi];
+    float v2 = -INFINITY;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      const int j = cg * CPL + c;
+      if (j < N && j != bi && !(bflat && s_fc[j])) v2 = max_sel(v2, sL[line * P + j]);
+    }
+    v2 = group_max(v2);
+    if (cg == 0 && line < N && !fr) atomicAdd(&s_cnt[bi], 1);
+    __syncthreads();
+    bool good = true;
+    if (line < N) {
+      const float lb = __logf(bv);
+      good = lb - v2 > TRK_MARGIN && fabsf(bv - 0.3f) > 1e-2f && s_cnt[line] <= 1;   // NaN: not good
+    }
+    if (!__syncthreads_and(good)) return;
+  }
+  if (n_iters > 0 && cg == 0 && line < N)
+    __hip_atomic_store(sg + line, bi | TRK_READY | (fr ? TRK_FLAT : 0) | (bv > 0.3f ? TRK_CONF : 0), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The matching half of the tracking loop (model.py:233-252), workgroup b < clips for clip b.  C: cost between
 // the unpermuted frames t-1 and t, [clip][T-1][N][N]; alive [clip][T][N] (null: all alive).  Writes, for
 // t >= 1, perm32 / perm64 / matched / alive_out at [clip][t][i] (t = 0: identity, 0, alive of frame 0).
 // The next frame pair's cost block is loaded into registers while the current step runs.
+// sig [clip][T][N] (nullable): the workgroups after the first `clips` match the frame pairs ahead of the loop (frame
+// TRK_AHEAD of every clip first), and a step whose match is there and decides takes it.  The loop's waves issue first.
 template <int CPL>
 __global__ void __launch_bounds__(64 * CPL)
 track_sequence_kernel(const float* __restrict__ C, const float* __restrict__ alive, int* __restrict__ perm32,
                       int64_t* __restrict__ perm64, float* __restrict__ matched, float* __restrict__ alive_out,
-                      int T, int N, int n_iters, float inv_t) {
+                      int* sig, int clips, int T, int N, int n_iters, float inv_t) {
   using S = SkTile<CPL>;
   constexpr int NC = S::NC, P = S::P;
   __shared__ float sL[NC * P];     // log_alpha of the current step
   __shared__ float sC[NC * P];     // cost block of the current frame pair (rows of the unpermuted frame)
   __shared__ int sperm[NC];        // perm of the previous step (rows of the tracked frame t-1)
   __shared__ float salive[NC];     // alive of the tracked frame t-1
-  const int64_t b = blockIdx.x;
+  __shared__ int s_cnt[NC];        // occurrences of the frame's rows
+  __shared__ int s_sig[8 * NC];    // frames tb .. tb + 7: sig and alive
+  __shared__ float s_al[8 * NC];
   const int tid = threadIdx.x, line = (tid >> 6) * 8 + ((tid & 63) >> 3), cg = tid & 7;
+  if ((int)blockIdx.x >= clips) {
+    const int64_t u = (int)blockIdx.x - clips, b = u % clips, t = TRK_AHEAD + u / clips;
+    track_pair<CPL>(C + (b * (T - 1) + t - 1) * N * N, sig + (b * T + t) * N, sL, sperm, s_cnt, line, cg, N, n_iters,
+                    inv_t);
+    return;
+  }
+  __builtin_amdgcn_s_setprio(3);
+  const int64_t b = blockIdx.x;
   const int64_t base = b * T * N;
   if (cg == 0 && line < N) {
     const float al = alive ? alive[base + line] : 1.f;
@@ -525,12 +620,67 @@ track_sequence_kernel(const float* __restrict__ C, const float* __restrict__ ali
       pf[c] = (line < N && j < N) ? ct[j] : 0.f;
     }
   };
+  int pft = 1;      // the frame pf belongs to
   if (T > 1) prefetch(1);
-  for (int t = 1; t < T; ++t) {
+  // the matches found ahead for 8 frames, one per lane of the row's group
+  int tb = 1, sg = 0;
+  float sa = 1.f;
+  auto fetch = [&](int t0) {
+    sg = 0;
+    if (line < N && t0 + cg < T) {
+      const int64_t o = base + (int64_t)(t0 + cg) * N + line;
+      sg = __hip_atomic_load(sig + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sa = alive ? alive[o] : 1.f;
+    }
+  };
+  auto stash = [&](int t0) {
+    s_sig[cg * NC + line] = sg;
+    s_al[cg * NC + line] = sa;
+    tb = t0;
+  };
+  if (sig) {
+    sg = 0;
+    stash(1);
+  }
+  auto put = [&](int t, int bi, float a1, bool conf) {     // (lanes cg == 0, line < N)
+    const int64_t o = base + (int64_t)t * N + line;
+    perm32[o] = bi;
+    if (perm64) perm64[o] = bi;
+    matched[o] = (salive[line] > 0.5f ? 1.f : 0.f) * (a1 > 0.5f ? 1.f : 0.f) * (conf ? 1.f : 0.f);
+    if (alive_out) alive_out[o] = a1;
+    salive[line] = a1;
+    sperm[line] = bi;
+  };
+  auto store_c = [&]() {
 #pragma unroll
     for (int c = 0; c < CPL; ++c) sC[line * P + cg * CPL + c] = pf[c];
-    __syncthreads();   // sC complete; the previous step's sperm / salive updates visible
+  };
+  for (int t = 1; t < T; ++t) {
+    if (sig && t - tb == 8) stash(t);     // (fetched on the way)
+    if (pft == t) store_c();
+    if (cg == 0) s_cnt[line] = 0;
+    __syncthreads();   // sC and the stash complete; the previous step's sperm / salive updates visible
+    if (sig && t - tb == 3) fetch(tb + 8);
+    const int* ss = s_sig + (t - tb) * NC;
+    if (sig && (ss[0] & TRK_READY)) {
+      const int pr = line < N ? sperm[line] : 0, sv = ss[pr], own = ss[line];
+      const float a1 = s_al[(t - tb) * NC + (sv & TRK_IDX)];
+      if (cg == 0 && line < N && !(sv & TRK_FLAT)) atomicAdd(&s_cnt[pr], 1);
+      __syncthreads();
+      // every row that is not flat once
+      const bool good = line >= N || ((own & TRK_READY) && ((own & TRK_FLAT) || s_cnt[line] == 1));
+      if (__syncthreads_and(good)) {
+        if (cg == 0 && line < N) put(t, sv & TRK_IDX, a1, sv & TRK_CONF);
+        continue;        // (the next step's first barrier orders these updates)
+      }
+    }
+    if (pft != t) {
+      prefetch(t);
+      store_c();
+      __syncthreads();
+    }
     if (t + 1 < T) prefetch(t + 1);
+    pft = t + 1;
     const float* src = sC + (line < N ? sperm[line] : 0) * P;
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
@@ -538,21 +688,20 @@ track_sequence_kernel(const float* __restrict__ C, const float* __restrict__ ali
       sL[line * P + j] = (line < N && j < N) ? la_of(src[j], inv_t) : -INFINITY;
     }
     __syncthreads();
-    sinkhorn_lds<CPL>(sL, n_iters, line, cg);
+    // while the pairs are being matched, look again after each step (late: the rounds that hide the loads)
+    const bool look = sig && t < 3 * TRK_AHEAD;
+    const int late = look ? min(n_iters, 4) : 0;
+    sinkhorn_lds<CPL>(sL, n_iters - late, line, cg);
+    if (look) {
+      fetch(t + 1);
+      sinkhorn_lds<CPL>(sL, late, line, cg);
+    }
     float bv;
     int bi;
     argmax_row<CPL>(sL, N, line, cg, bv, bi);
     __syncthreads();   // every lane has read sperm, sC and sL
-    if (cg == 0 && line < N) {
-      const int64_t o = base + (int64_t)t * N;
-      const float a1 = alive ? alive[o + bi] : 1.f;
-      perm32[o + line] = bi;
-      if (perm64) perm64[o + line] = bi;
-      matched[o + line] = (salive[line] > 0.5f ? 1.f : 0.f) * (a1 > 0.5f ? 1.f : 0.f) * (bv > 0.3f ? 1.f : 0.f);
-      if (alive_out) alive_out[o + line] = a1;
-      salive[line] = a1;
-      sperm[line] = bi;
-    }
+    if (cg == 0 && line < N) put(t, bi, alive ? alive[base + (int64_t)t * N + bi] : 1.f, bv > 0.3f);
+    if (look) stash(t + 1);
   }
 }
 
@@ -683,12 +832,12 @@ static int launch_cost_dt(int dtype, const TrackCostArgs& a, hipStream_t st) {
   }
 }
 
-static int clamp_rows(const float* x, float* y, int64_t n, hipStream_t st) {
+static int clamp_rows(const float* x, float* y, int64_t n, int* z, int64_t nz, hipStream_t st) {
   if (n == 0) return 0;
   if (n % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)y & 15) == 0)
-    hipLaunchKernelGGL(trk_clamp_kernel<4>, dim3(blocks256(n / 4)), dim3(256), 0, st, x, y, n);
+    hipLaunchKernelGGL(trk_clamp_kernel<4>, dim3(blocks256(n / 4)), dim3(256), 0, st, x, y, n, z, nz);
   else
-    hipLaunchKernelGGL(trk_clamp_kernel<1>, dim3(blocks256(n)), dim3(256), 0, st, x, y, n);
+    hipLaunchKernelGGL(trk_clamp_kernel<1>, dim3(blocks256(n)), dim3(256), 0, st, x, y, n, z, nz);
   HCLSM_LAUNCH_CHECK();
   return 0;
 }
@@ -719,7 +868,7 @@ static float inv_temperature(float temperature) { return 1.f / (temperature > 1e
 static size_t al256t(size_t v) { return (v + 255) / 256 * 256; }
 
 struct SeqWs {
-  size_t s, uv, c, perm, matched, gi, gh, total;
+  size_t s, uv, c, perm, matched, sig, gi, gh, total;
 };
 
 static SeqWs seq_ws(int64_t B, int64_t T, int64_t N, int64_t D, bool hidden) {
@@ -731,6 +880,7 @@ static SeqWs seq_ws(int64_t B, int64_t T, int64_t N, int64_t D, bool hidden) {
   w.c = o; o += al256t((size_t)B * (T > 0 ? T - 1 : 0) * N * N * 4);
   w.perm = o; o += al256t(R * 4);
   w.matched = o; o += al256t(R * 4);
+  w.sig = o; o += al256t(R * 4);
   if (hidden) {
     w.gi = o; o += al256t(R * 3 * D * 4);
     w.gh = o; o += al256t((size_t)B * N * 3 * D * 4);
@@ -773,8 +923,8 @@ extern "C" int hclsm_slot_track_cost(const float* slots_t, const float* slots_t1
   float* S = reinterpret_cast<float*>(ws);
   float* UV = reinterpret_cast<float*>(ws + al256t((size_t)R * D * 4));
   int rc;
-  if ((rc = clamp_rows(slots_t, S, FN * D, st))) return rc;
-  if ((rc = clamp_rows(slots_t1, S + FN * D, FN * D, st))) return rc;
+  if ((rc = clamp_rows(slots_t, S, FN * D, nullptr, 0, st))) return rc;
+  if ((rc = clamp_rows(slots_t1, S + FN * D, FN * D, nullptr, 0, st))) return rc;
   const int es = dtype == HCLSM_F32 ? 4 : 2;
   const char* W1 = reinterpret_cast<const char*>(params[0]);
   const float* b1 = reinterpret_cast<const float*>(params[1]);
@@ -903,9 +1053,19 @@ extern "C" int hclsm_slot_track_sequence(const float* slots, const float* alive,
   const int64_t R = batch * T * N;
   const int es = dtype == HCLSM_F32 ? 4 : 2;
   int rc;
+  // Match the pairs ahead of the loop while the loop's one workgroup per clip leaves compute units idle.  Whole call
+  // without / with, in us, for matches that decide and for weights that decide nothing (the loop does every step):
+  //   32 clips of 32 frames, 32 slots, D 192:  632 / 499 and 630 / 636;  256 clips: 2513 / 2446 and 2516 / 2508
+  //   one clip of 32 frames, 16 slots, D 64: 250 / 174 and 252 / 259;  128 slots, 8 frames, 1 clip: 633 / 574 and 636 / 656
+  //   256 clips of 64 slots, 16 frames: 2898 / 2991 and of 128 slots, 8 frames: 3252 / 3704 (two workgroups' tiles of
+  //   over 32 slots crowd a compute unit's LDS), hence half as many clips above 32 slots; 3 frames are run by the loop.
+  int cus = 0;
+  if ((rc = device_cus(&cus))) return rc;
+  const bool ahead = T >= 4 && batch <= (N <= 32 ? cus : cus / 2) && batch * T <= 0x7fffffffLL;
+  int* sig = reinterpret_cast<int*>(ws + L.sig);
   if (T > 1) {
     // pair MLP over every (t-1, t) frame pair: U = W1a s + b1 and V = W1b s for every node row
-    if ((rc = clamp_rows(slots, S, R * D, st))) return rc;
+    if ((rc = clamp_rows(slots, S, R * D, ahead ? sig : nullptr, R, st))) return rc;
     const char* W1 = reinterpret_cast<const char*>(params[0]);
     if ((rc = linear_rows(S, D, HCLSM_F32, W1, 3 * D, reinterpret_cast<const float*>(params[1]), nullptr, 0, UV,
                           2 * D, HCLSM_F32, R, D, D, 0, 0, nullptr, nullptr, 0.f, nullptr, 0, nullptr, 1, dtype, st)))
@@ -930,8 +1090,9 @@ extern "C" int hclsm_slot_track_sequence(const float* slots, const float* alive,
   const float inv_t = inv_temperature(temperature);
   rc = with_tile(N, [&](auto cpl) {
     constexpr int CPL = decltype(cpl)::value;
-    hipLaunchKernelGGL((track_sequence_kernel<CPL>), dim3((unsigned)batch), dim3(64 * CPL), 0, st, C, alive, P, perm,
-                       M, alive_out, (int)T, (int)N, (int)n_iters, inv_t);
+    const unsigned pairs = ahead ? (unsigned)(batch * (T - TRK_AHEAD)) : 0u;
+    hipLaunchKernelGGL((track_sequence_kernel<CPL>), dim3((unsigned)batch + pairs), dim3(64 * CPL), 0, st, C, alive, P,
+                       perm, M, alive_out, ahead ? sig : nullptr, (int)batch, (int)T, (int)N, (int)n_iters, inv_t);
     HCLSM_LAUNCH_CHECK();
     return 0;
   });
