@@ -48,6 +48,8 @@ struct TrackCostArgs {
   int64_t pairs;       // F * N * N
   int N, D;
   int nt, tstride, fboff;   // cost frame f pairs node frames fa = (f / nt) * tstride + f % nt and fa + fboff
+  // weight-resident kernel: a unit is one of `parts` row ranges of a group of 32 staged rows (cost_units)
+  int frames, units, parts;
 };
 
 template <int DT, int NW, int KC>
@@ -156,25 +158,48 @@ track_cost_kernel(TrackCostArgs a) {
 }
 
 // Weight-resident variant for 16-bit operands and D <= 192 (the pair tiles of the tiny and small presets):
-// a persistent workgroup stages W1c and W2 in LDS once, then walks blocks of 32 NW pairs.  The MFMAs take
+// a persistent workgroup stages W1c and W2 in LDS once.  It then walks units: the 32 rows of S and V of the later
+// slots in LDS (rows of one frame, or of 2 or 4 frames of at most 16 or 8 slots; the next unit's rows are loaded
+// while this one's pairs run), against a range of the earlier slots.  A wave takes 4 earlier x 8 later slots at a
+// time as two 16-pair tiles that share each weight fragment and each later row read from LDS.  The MFMAs take
 // the weights as the A operand and the pairs as the B operand, so lane (g, li) of a 16-output tile holds
-// outputs 4g .. 4g+3 of pair li: the U / V epilogue reads float4s, and the first layer's accumulators are,
+// outputs 4g .. 4g+3 of pair li: U_i + V_j in float4s starts the accumulators, and these are,
 // without leaving registers, the second layer's B operand, with W2's columns stored in the matching order
-// (positions 8g .. 8g+7 of a 32-wide block hold k = 4g .. 4g+3 and 16 + 4g .. 16 + 4g+3).  Two 16-pair
-// tiles per wave share each weight fragment read from LDS.
+// (positions 8g .. 8g+7 of a 32-wide block hold k = 4g .. 4g+3 and 16 + 4g .. 16 + 4g+3).
+// 2.06 M pairs at D 192 in bf16 (190 GFLOP): 268 us, 710 TFLOP/s; 466 us with every pair's rows of S and V read from
+// L2 (3.1 GB) and U and V added after the products.  What is left is spread: of a wave's 8.4 us per 32 pairs, LDS reads
+// take 3, loads of X and U 2.6, MFMAs 2.4 and vector instructions 2.4, and the registers allow two waves a SIMD to
+// overlap them (three waves with spills: 413 us; operands formed during the products, spilling: 311 us).
+template <int DT>
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  if constexpr (DT == HCLSM_BF16)
+    return pack_bf16x2(lo, hi);
+  else
+    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) |
+           (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16;
+}
+
+// max(x, 0) in one instruction (fmaxf quiets its operand first); NaN gives 0, as fmaxf does
+__device__ __forceinline__ float relu1(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, INFINITY); }
+
+constexpr int TRK_ROWS = 32;     // staged rows of a unit
+
 template <int DT, int D, int NW>
 __global__ void __launch_bounds__(64 * NW)
 track_cost_res_kernel(TrackCostArgs a) {
   using A = MM<DT>;
   using T = typename A::T;
   static_assert(DT != HCLSM_F32 && D % 64 == 0 && D <= 192, "16-bit operands, D a multiple of 64 up to 192");
-  constexpr int NTH = 64 * NW, PT = 2, BLK = 16 * PT * NW;
-  constexpr int D4 = D / 4, PW = D + 8, NT = D / 16, NT2 = D4 / 16, NKB = D / 32;
+  constexpr int NTH = 64 * NW, PT = 2;
+  constexpr int D4 = D / 4, PW = D + 8, PY = D + 4, NT = D / 16, NT2 = D4 / 16, NKB = D / 32;
+  constexpr int NS = 2 * TRK_ROWS * D4 / NTH;          // float4s of a unit's rows per thread
+  static_assert(2 * TRK_ROWS * D4 % NTH == 0, "whole float4s");
   extern __shared__ __align__(16) unsigned char smem[];
   T* sW1 = reinterpret_cast<T*>(smem);                 // [D][PW] W1c, natural k order
   T* sW2 = sW1 + D * PW;                               // [D4][PW] W2, k permuted within 32-wide blocks
   float* sb2 = reinterpret_cast<float*>(sW2 + D4 * PW);
   float* sw3 = sb2 + D4;
+  float* sY = sw3 + D4;                                // [2][TRK_ROWS][PY] rows of S, rows of V
   const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63, g = lane >> 4, li = lane & 15;
   {
     const T* W1 = reinterpret_cast<const T*>(a.W1);
@@ -195,131 +220,162 @@ track_cost_res_kernel(TrackCostArgs a) {
       sw3[u] = a.w3[u];
     }
   }
-  __syncthreads();
   const int N = a.N;
-  const int64_t NN = (int64_t)N * N;
-  auto nodes_of = [&](int64_t p, int64_t& ra, int64_t& rb) {
-    p = p < a.pairs ? p : a.pairs - 1;
-    const int64_t f = p / NN;
-    const int rem = (int)(p - f * NN);
-    const int i = rem / N, j = rem - i * N;
-    const int64_t q = f / a.nt;
-    const int64_t fa = q * a.tstride + (f - q * a.nt);
-    ra = fa * N + i;
-    rb = (fa + a.fboff) * N + j;
+  const int nct = (N + 7) / 8, nrg = (N + 3) / 4;      // column tiles of 8, row groups of 4
+  const int FP = nct == 1 ? 4 : nct == 2 ? 2 : 1;      // frames of a unit
+  const int CG = FP > 1 ? 1 : (nct + 3) / 4;           // units across a frame's columns
+  const int rgp = (nrg + a.parts - 1) / a.parts;
+  auto frame_a = [&](int f) {                          // first node row of the earlier frame
+    const int q = f / a.nt;
+    return ((int64_t)q * a.tstride + (f - q * a.nt)) * N;
   };
-  const int64_t nblk = (a.pairs + BLK - 1) / BLK;
-  for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
-    const int64_t pw = blk * BLK + (int64_t)wid * 16 * PT;
-    int64_t ra[PT], rb[PT];
+  f32x4 nx[NS];
+  auto stage_load = [&](int u) {
+    const int uf = u / a.parts, fg = uf / CG, cg = uf - fg * CG;
 #pragma unroll
-    for (int pt = 0; pt < PT; ++pt) nodes_of(pw + 16 * pt + li, ra[pt], rb[pt]);
-    // ---- first layer: acc[pt][t] = W1c rows 16t.. x |a - b| of the tile's pairs
-    f32x4 acc[PT][NT];
+    for (int v = 0; v < NS; ++v) {
+      const int e = tid + v * NTH, r = e / D4, c = e - r * D4, w = r / TRK_ROWS, s = r - w * TRK_ROWS;
+      const int fr = FP > 1 ? s / (8 * nct) : 0;
+      const int j = FP > 1 ? s - fr * 8 * nct : cg * TRK_ROWS + s;
+      const int f = min(fg * FP + fr, a.frames - 1);
+      const int64_t rb = frame_a(f) + (int64_t)a.fboff * N + min(j, N - 1);
+      nx[v] = *reinterpret_cast<const f32x4*>(w ? a.UV + rb * 2 * D + D + 4 * c : a.S + rb * D + 4 * c);
+    }
+  };
+  // consecutive units: the rows of one unit's later frame are the next one's earlier rows, in this XCD's L2 by then
+  const int u1 = (int)((int64_t)(blockIdx.x + 1) * a.units / gridDim.x);
+  int u = (int)((int64_t)blockIdx.x * a.units / gridDim.x);
+  if (u < u1) stage_load(u);
+  for (; u < u1; ++u) {
+    __syncthreads();       // the weights are in place; the previous unit's rows have been read
 #pragma unroll
-    for (int pt = 0; pt < PT; ++pt)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[pt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // raw rows of the next k-block are loaded while the current one is multiplied
-    float4 xr[PT][4];
-    auto load_k = [&](int kb) {
+    for (int v = 0; v < NS; ++v) {
+      const int e = tid + v * NTH, r = e / D4, c = e - r * D4;
+      *reinterpret_cast<f32x4*>(sY + r * PY + 4 * c) = nx[v];
+    }
+    __syncthreads();
+    bool staged = u + 1 >= u1;
+    const int uf = u / a.parts, part = u - uf * a.parts, fg = uf / CG, cg = uf - fg * CG;
+    const int ntile = FP > 1 ? FP * nct : min(4, nct - 4 * cg);
+    const int rg0 = part * rgp, nr = min(rgp, nrg - rg0);
+    const int items = ntile * max(nr, 0), per = (items + NW - 1) / NW;
+    for (int it = wid * per; it < min((wid + 1) * per, items); ++it) {
+      const int rgi = it / ntile, ct = it - rgi * ntile;
+      const int fr = FP > 1 ? ct / nct : 0;
+      const int f = fg * FP + fr;
+      const int j = (FP > 1 ? ct - fr * nct : 4 * cg + ct) * 8 + (li & 7);
+      const int64_t fa = frame_a(min(f, a.frames - 1));
+      int i[PT];
+      const float *X[PT], *U[PT];
 #pragma unroll
       for (int pt = 0; pt < PT; ++pt) {
-        const float* xa = a.S + ra[pt] * D + kb + 8 * g;
-        const float* xb = a.S + rb[pt] * D + kb + 8 * g;
-        xr[pt][0] = *reinterpret_cast<const float4*>(xa);
-        xr[pt][1] = *reinterpret_cast<const float4*>(xa + 4);
-        xr[pt][2] = *reinterpret_cast<const float4*>(xb);
-        xr[pt][3] = *reinterpret_cast<const float4*>(xb + 4);
+        i[pt] = (rg0 + rgi) * 4 + 2 * pt + (li >> 3);
+        const int64_t ra = fa + min(i[pt], N - 1);
+        X[pt] = a.S + ra * D + 8 * g;
+        U[pt] = a.UV + ra * 2 * D + 4 * g;
       }
-    };
-    load_k(0);
-#pragma unroll 1
-    for (int kb = 0; kb < D; kb += 32) {
-      T op[PT][8];
+      const float* yr = sY + (8 * ct + (li & 7)) * PY;
+      const float* vr = yr + TRK_ROWS * PY + 4 * g;
+      // ---- first layer: acc[pt][t] = U_i + V_j + W1c rows 16t.. x |a - b| of the tile's pairs
+      float4 xr[2][PT][2];
+      auto load_k = [&](int kb, int s) {
 #pragma unroll
-      for (int pt = 0; pt < PT; ++pt) {
-        const float4 x0 = xr[pt][0], x1 = xr[pt][1], y0 = xr[pt][2], y1 = xr[pt][3];
-        op[pt][0] = A::fromf(fabsf(x0.x - y0.x)); op[pt][1] = A::fromf(fabsf(x0.y - y0.y));
-        op[pt][2] = A::fromf(fabsf(x0.z - y0.z)); op[pt][3] = A::fromf(fabsf(x0.w - y0.w));
-        op[pt][4] = A::fromf(fabsf(x1.x - y1.x)); op[pt][5] = A::fromf(fabsf(x1.y - y1.y));
-        op[pt][6] = A::fromf(fabsf(x1.z - y1.z)); op[pt][7] = A::fromf(fabsf(x1.w - y1.w));
-      }
-      if (kb + 32 < D) load_k(kb + 32);
+        for (int pt = 0; pt < PT; ++pt) {
+          xr[s][pt][0] = *reinterpret_cast<const float4*>(X[pt] + 32 * kb);
+          xr[s][pt][1] = *reinterpret_cast<const float4*>(X[pt] + 32 * kb + 4);
+        }
+      };
+      load_k(0, 0);
+      load_k(1, 1);
+      f32x4 acc[PT][NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int pt = 0; pt < PT; ++pt) acc[pt][t] = *reinterpret_cast<const f32x4*>(U[pt] + 16 * t);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        T wf[8];
-        frag_load<DT>(sW1 + (16 * t + li) * PW + kb + 8 * g, wf);
+        const f32x4 v4 = *reinterpret_cast<const f32x4*>(vr + 16 * t);
 #pragma unroll
-        for (int pt = 0; pt < PT; ++pt) acc[pt][t] = frag_mma<DT>(wf, op[pt], acc[pt][t]);
+        for (int pt = 0; pt < PT; ++pt) acc[pt][t] = acc[pt][t] + v4;
+        if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    // ---- epilogue: h = ReLU(acc + U_i + V_j) for outputs 16t + 4g + rr of pair li
-    // (in groups of 3 tiles: the scheduler would otherwise hoist every load of the epilogue at once)
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int pt = 0; pt < PT; ++pt) {
-      const float* U = a.UV + ra[pt] * 2 * D + 4 * g;
-      const float* V = a.UV + rb[pt] * 2 * D + D + 4 * g;
+      for (int kb = 0; kb < NKB; ++kb) {
+        const float4 y0 = *reinterpret_cast<const float4*>(yr + 32 * kb + 8 * g);
+        const float4 y1 = *reinterpret_cast<const float4*>(yr + 32 * kb + 8 * g + 4);
+        T op[PT][8];
 #pragma unroll
-      for (int t0 = 0; t0 < NT; t0 += 3) {
-#pragma unroll
-        for (int t = t0; t < t0 + 3 && t < NT; ++t) {
-          const float4 u4 = *reinterpret_cast<const float4*>(U + 16 * t);
-          const float4 v4 = *reinterpret_cast<const float4*>(V + 16 * t);
-          acc[pt][t][0] = fmaxf(acc[pt][t][0] + u4.x + v4.x, 0.f);
-          acc[pt][t][1] = fmaxf(acc[pt][t][1] + u4.y + v4.y, 0.f);
-          acc[pt][t][2] = fmaxf(acc[pt][t][2] + u4.z + v4.z, 0.f);
-          acc[pt][t][3] = fmaxf(acc[pt][t][3] + u4.w + v4.w, 0.f);
+        for (int pt = 0; pt < PT; ++pt) {
+          const float4 x0 = xr[kb & 1][pt][0], x1 = xr[kb & 1][pt][1];
+          *reinterpret_cast<uint4*>(op[pt]) =
+              make_uint4(pack2<DT>(fabsf(x0.x - y0.x), fabsf(x0.y - y0.y)),
+                         pack2<DT>(fabsf(x0.z - y0.z), fabsf(x0.w - y0.w)),
+                         pack2<DT>(fabsf(x1.x - y1.x), fabsf(x1.y - y1.y)),
+                         pack2<DT>(fabsf(x1.z - y1.z), fabsf(x1.w - y1.w)));
         }
-        __builtin_amdgcn_sched_barrier(0);
+        if (kb + 2 < NKB) load_k(kb + 2, kb & 1);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          T wf[8];
+          frag_load<DT>(sW1 + (16 * t + li) * PW + 32 * kb + 8 * g, wf);
+#pragma unroll
+          for (int pt = 0; pt < PT; ++pt) acc[pt][t] = frag_mma<DT>(wf, op[pt], acc[pt][t]);
+        }
+        __builtin_amdgcn_sched_barrier(0);    // (no further: the loads of all steps at once do not fit the registers)
       }
-    }
-    // ---- second layer: k-block kb takes tiles 2kb (k = 32kb + 4g + e) and 2kb + 1 (32kb + 16 + 4g + e)
-    f32x4 acc2[PT][NT2];
-#pragma unroll
-    for (int pt = 0; pt < PT; ++pt)
-#pragma unroll
-      for (int t = 0; t < NT2; ++t) acc2[pt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-      T hb[PT][8];
+      if (!staged) {       // (after this item's own loads, so that they are not waited for in their place)
+        stage_load(u + 1);
+        staged = true;
+      }
+      // ---- second layer: k-block kb takes tiles 2kb (k = 32kb + 4g + e) and 2kb + 1 (32kb + 16 + 4g + e)
+      f32x4 acc2[PT][NT2];
 #pragma unroll
       for (int pt = 0; pt < PT; ++pt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          hb[pt][e] = A::fromf(acc[pt][2 * kb][e]);
-          hb[pt][4 + e] = A::fromf(acc[pt][2 * kb + 1][e]);
+        for (int t = 0; t < NT2; ++t) acc2[pt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb) {
+        T hb[PT][8];
+#pragma unroll
+        for (int pt = 0; pt < PT; ++pt) {
+          const f32x4 h0 = acc[pt][2 * kb], h1 = acc[pt][2 * kb + 1];
+          *reinterpret_cast<uint4*>(hb[pt]) =
+              make_uint4(pack2<DT>(relu1(h0[0]), relu1(h0[1])), pack2<DT>(relu1(h0[2]), relu1(h0[3])),
+                         pack2<DT>(relu1(h1[0]), relu1(h1[1])), pack2<DT>(relu1(h1[2]), relu1(h1[3])));
         }
 #pragma unroll
-      for (int t = 0; t < NT2; ++t) {
-        T wf[8];
-        frag_load<DT>(sW2 + (16 * t + li) * PW + 32 * kb + 8 * g, wf);
+        for (int t = 0; t < NT2; ++t) {
+          T wf[8];
+          frag_load<DT>(sW2 + (16 * t + li) * PW + 32 * kb + 8 * g, wf);
 #pragma unroll
-        for (int pt = 0; pt < PT; ++pt) acc2[pt][t] = frag_mma<DT>(wf, hb[pt], acc2[pt][t]);
+          for (int pt = 0; pt < PT; ++pt) acc2[pt][t] = frag_mma<DT>(wf, hb[pt], acc2[pt][t]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // ---- score of pair li: sum over the second layer's outputs 16t + 4g + rr, then over the 4 lane groups
+#pragma unroll
+      for (int pt = 0; pt < PT; ++pt) {
+        float sum = 0.f;
+#pragma unroll
+        for (int t = 0; t < NT2; ++t)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) {
+            const int o = 16 * t + 4 * g + rr;
+            sum = fmaf(relu1(acc2[pt][t][rr] + sb2[o]), sw3[o], sum);
+          }
+        sum = rows4_sum(sum);
+        if (g == 0 && i[pt] < N && j < N && f < a.frames) {
+          float s = sum + a.b3[0];
+          if (a.alive_a) {
+            s = s - (a.alive_a[fa + i[pt]] < 0.5f ? TRK_PENALTY : 0.f);
+            s = s - (a.alive_b[fa + (int64_t)a.fboff * N + j - a.boff] < 0.5f ? TRK_PENALTY : 0.f);
+          }
+          a.cost[((int64_t)f * N + i[pt]) * N + j] = -s;
+        }
       }
     }
-    // ---- score of pair li: sum over the second layer's outputs 16t + 4g + rr, then over the 4 lane groups
-#pragma unroll
-    for (int pt = 0; pt < PT; ++pt) {
-      float part = 0.f;
-#pragma unroll
-      for (int t = 0; t < NT2; ++t)
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int o = 16 * t + 4 * g + rr;
-          part = fmaf(fmaxf(acc2[pt][t][rr] + sb2[o], 0.f), sw3[o], part);
-        }
-      part = rows4_sum(part);
-      const int64_t p = pw + 16 * pt + li;
-      if (g == 0 && p < a.pairs) {
-        float s = part + a.b3[0];
-        if (a.alive_a) {
-          s = s - (a.alive_a[ra[pt]] < 0.5f ? TRK_PENALTY : 0.f);
-          s = s - (a.alive_b[rb[pt] - a.boff] < 0.5f ? TRK_PENALTY : 0.f);
-        }
-        a.cost[p] = -s;
-      }
-    }
+    if (!staged) stage_load(u + 1);
   }
 }
 
@@ -792,17 +848,36 @@ static int launch_cost_kc(const TrackCostArgs& a, hipStream_t st) {
   return 0;
 }
 
+// Row ranges per group of staged rows: the whole ranges' time on `grid` workgroups, in turns of 4 x 8 pairs per wave
+// plus one for a unit's own start, is least
+static void cost_units(TrackCostArgs& a, int64_t frames, int NW, int grid) {
+  const int64_t nct = (a.N + 7) / 8, nrg = (a.N + 3) / 4;
+  const int64_t FP = nct == 1 ? 4 : nct == 2 ? 2 : 1, CG = FP > 1 ? 1 : (nct + 3) / 4;
+  const int64_t groups = (frames + FP - 1) / FP * CG, tiles = FP > 1 ? FP * nct : (nct < 4 ? nct : 4);
+  int64_t best = -1;
+  for (int64_t p = 1; p <= nrg && p <= 64; ++p) {
+    const int64_t items = (nrg + p - 1) / p * tiles;
+    const int64_t t = (groups * p + grid - 1) / grid * ((items + NW - 1) / NW + 1);
+    if (best >= 0 && t >= best) continue;
+    best = t;
+    a.parts = (int)p;
+  }
+  a.frames = (int)frames;
+  a.units = (int)(groups * a.parts);
+}
+
 template <int DT, int D, int NW>
-static int launch_cost_res(const TrackCostArgs& a, hipStream_t st) {
+static int launch_cost_res(TrackCostArgs a, hipStream_t st) {
   using T = typename MM<DT>::T;
-  constexpr size_t lds = ((size_t)D * (D + 8) + (size_t)(D / 4) * (D + 8)) * sizeof(T) + (size_t)(D / 4) * 8;
+  constexpr size_t lds = ((size_t)D * (D + 8) + (size_t)(D / 4) * (D + 8)) * sizeof(T) + (size_t)(D / 4) * 8 +
+                         (size_t)2 * TRK_ROWS * (D + 4) * 4;
   static std::atomic<int> setup[HCLSM_MAX_DEVICES];   // resident workgroups per device (persistent kernel)
   int grid = 0;
   const int se = device_launch_setup(reinterpret_cast<const void*>(&track_cost_res_kernel<DT, D, NW>), 64 * NW, lds,
                                      (int)TRK_LDS_MAX, setup, &grid);
   if (se) return se;
-  const int64_t nblk = (a.pairs + 32 * NW - 1) / (32 * NW);
-  const unsigned g = (unsigned)(nblk < grid ? nblk : grid);
+  cost_units(a, a.pairs / ((int64_t)a.N * a.N), NW, grid);
+  const unsigned g = (unsigned)(a.units < grid ? a.units : grid);
   hipLaunchKernelGGL((track_cost_res_kernel<DT, D, NW>), dim3(g), dim3(64 * NW), lds, st, a);
   HCLSM_LAUNCH_CHECK();
   return 0;
