@@ -58,6 +58,8 @@ template <> struct MM<HCLSM_F32> {
   static __device__ __forceinline__ T fromf(float v) { return v; }
 };
 
+// max(x, 0) in one instruction (fmaxf quiets its operand first); NaN gives 0, as fmaxf does
+__device__ __forceinline__ float relu1(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, INFINITY); }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + __expf(-x)); }
 __device__ __forceinline__ float tanh_f(float x) {
   // 1 - 2/(e^{2x}+1): saturates cleanly to +-1 at both ends

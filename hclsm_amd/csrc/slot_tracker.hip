@@ -179,9 +179,6 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
            (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16;
 }
 
-// max(x, 0) in one instruction (fmaxf quiets its operand first); NaN gives 0, as fmaxf does
-__device__ __forceinline__ float relu1(float x) { return __builtin_amdgcn_fmed3f(x, 0.f, INFINITY); }
-
 constexpr int TRK_ROWS = 32;     // staged rows of a unit
 
 template <int DT, int D, int NW>
