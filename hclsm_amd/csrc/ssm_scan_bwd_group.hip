@@ -426,10 +426,13 @@ int bwd_group(int mode, const void* x, const void* dt, const float* A_log, const
   HCLSM_BG(DT_, SG_, HCLSM_SCAN_BLOCK) HCLSM_BG(DT_, SG_, BWD_BLOCK_GATE)
   int cus = 0;
   if (int rc = device_cus(&cus)) return rc;
-  // 8 states a lane fill a CU's 16 wave slots (4 per SIMD) for d_state 32 and 64; 16 a lane (12 slots) where groups of 8
-  // do not: d_state 48 in bf16, us 16 | 8 a lane: 1024 x 16 x 384 353 | 407, block 372 | 499, but 16 x 128 x 512 in fp32
-  // 262 | 182 (few workgroups, and no matrix core); past 64 states 8 a lane would need more than 8 waves.
-  const bool wide = S > 8 * BG_MAX_WAVES || (dtype == HCLSM_BF16 && S == 48 && N * ((Dn + 63) / 64) >= 4 * (int64_t)cus);
+  // A CU has 16 wave slots at 8 states a lane (4 waves per SIMD) and 12 at 16 a lane.  Workgroups of S/8 waves that do
+  // not divide 16 leave slots empty, 4 of them at d_state 48, where S/16 = 3 waves divide 12: us 16 | 8 a lane in bf16,
+  // 1024 x 16 x 384: 353 | 407, block 372 | 499.  With few workgroups the slots are empty anyway, and fp32 has no matrix
+  // core to take the wider lane's products: 16 x 128 x 512 in fp32 262 | 182.  32 and 64 states fill the slots at 8 a
+  // lane; past 64 states 8 a lane would need more than 8 waves.
+  const bool gaps = S % 16 == 0 && 16 % (S / 8) != 0;
+  const bool wide = S > 8 * BG_MAX_WAVES || (dtype == HCLSM_BF16 && gaps && N * ((Dn + 63) / 64) >= 4 * (int64_t)cus);
   if (wide) {
     if (dtype == HCLSM_BF16) { HCLSM_BG_M(HCLSM_BF16, 16) }
     else { HCLSM_BG_M(HCLSM_F32, 16) }
