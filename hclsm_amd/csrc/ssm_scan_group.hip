@@ -270,7 +270,7 @@ static int group_mode(int mode, const void* x, const void* dt, const float* A_lo
 int scan_fwd_group(int mode, const void* x, const void* dt, const float* A_log, const void* B, const void* C,
                    const float* Dskip, void* y, float* h_final, int64_t batch, int64_t T, int64_t Dn, int64_t S,
                    int dtype, hipStream_t st, ScanEpi epi) {
-  if (S % 8 != 0 || S < 16 || S > 8 * GRP_MAX_WAVES) return HCLSM_ERR_UNSUPPORTED;
+  if (S % 8 != 0 || S < 24 || S > 8 * GRP_MAX_WAVES) return HCLSM_ERR_UNSUPPORTED;
   if (dtype != HCLSM_BF16 && dtype != HCLSM_F32) return HCLSM_ERR_UNSUPPORTED;
   const int64_t es = dtype == HCLSM_F32 ? 4 : 2;
   if (T * Dn * es >= 0x7fffffffLL || T * S * es >= 0x7fffffffLL) return HCLSM_ERR_UNSUPPORTED;
@@ -282,11 +282,10 @@ int scan_fwd_group(int mode, const void* x, const void* dt, const float* A_log, 
   // 16 states a lane on the matrix core from four waves a CU on; below, 8 a lane double the waves (us, 16 | 8):
   // 128 x 16 x 256, S 32 (1024 waves) 10.8 | 8.7; 64 x 1024 x 384, S 32 (768) 537 | 440; 256 x 16 x 256, S 64 (4096)
   // 17.6 | 19.1; 1024 x 64 x 384, S 32 (12288) 149 | 174.  In fp32 both are within 3% of each other past that, so 8
-  // is used throughout.  d_state 16: one lane per channel (ssm_scan.hip; in bf16 always, so that the forward with
-  // and without the backward's checkpoints stay the same kernel) unless the grid is small: fp32, one lane | 8 a lane,
-  // (3072 waves) 57.5 | 54.4 and (6144) 86 | 110.
-  const bool few = w16 <= (S == 16 ? 12 : 4) * (int64_t)cus;
-  if (S == 16 && (dtype != HCLSM_F32 || !few)) return HCLSM_ERR_UNSUPPORTED;
+  // is used throughout.  d_state 16 stays on one lane per channel (ssm_scan.hip): in bf16 so that the forward with and
+  // without the backward's checkpoints is the same kernel; in fp32 a forward on a small grid is faster here (869 x 77 x
+  // 64: 48.7 | 42.9) but a training step with the backward after it is not (213 | 233).
+  const bool few = w16 <= 4 * (int64_t)cus;
   if (dtype == HCLSM_F32)
     return group_mode<HCLSM_F32, 8>(mode, x, dt, A_log, B, C, Dskip, y, h_final, batch, T, Dn, S, st, epi);
   if (S % 16 != 0 || few)
