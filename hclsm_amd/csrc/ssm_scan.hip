@@ -763,7 +763,7 @@ static int scan_entry(int mode, const void* x, const void* dt, const float* A_lo
     return 0;
   }
   if (!x || !dt || !A_log || !B || !C || !y) return HCLSM_ERR_NULL;
-  {   // wide states (and small grids of d_state 16); the generic kernel takes what it refuses
+  {   // wide states; the generic kernel takes what it refuses
     const int r = scan_fwd_group(mode, x, dt, A_log, B, C, Dskip, y, h_final, batch, T, d_inner, d_state, dtype, st, epi);
     if (r != HCLSM_ERR_UNSUPPORTED) return r;
   }
