@@ -593,6 +593,7 @@ __device__ __forceinline__ void track_pair(const float* __restrict__ cf, int* __
   fc &= dpp_i<0x4e>(fc);
   fc &= dpp_i<0x141>(fc);
   if (cg == 0) s_fc[line] = fc;
+  __syncthreads();                          // every column has been looked at before a wave normalises its rows in place
   float bv = 0.f;
   int bi = 0;
   for (int done = 0; done < n_iters;) {
