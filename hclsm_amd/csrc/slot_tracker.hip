@@ -554,13 +554,21 @@ track_match_kernel(const float* __restrict__ cost, const float* __restrict__ ali
 //  - no decision is close: sig is written only if in every row the best entry is at least TRK_MARGIN (in log units)
 //    above the best one of another column (columns that are flat throughout are equal to the bit and count as one; the
 //    lowest wins in either order) and not near the 0.3 threshold, and the rows that are not flat take distinct columns.
-//    The rounding is 1e-7 of these values.
+// How far the two orders can be apart: the first row step is the same to the bit.  The first column step subtracts a
+// log-sum-exp of up to twice the cost clamp over the temperature (M), so a column may shift by one unit of fp32 there,
+// u = ulp(M): 1/32 at the default temperature of 0.05.  After it the largest entry of every column is at least -log N,
+// of every row at least -2 log N, and a later row (column) step lowers what is in a column (row) by at most log N more:
+// all later sums are of size log N and round by about 1e-6 (entries that lie far below do not come back in n_iters
+// steps).  log-sum-exp does not enlarge a shift, so two entries of a row move against each other by at most 2 u and a
+// log probability by at most 2 u, plus about 4e-6 a round.  track_order_safe asks for u <= 1/32 and at most 1024
+// rounds: 2 u = 0.0625 of the 0.1 in log units, 0.02 of the 0.03 at the threshold.  At a lower temperature the loop does
+// every step by itself (two orders of the same rows could then decide differently: 0.1 is less than a unit at 0.001).
 // It gives up after TRK_EARLY rounds if the decisions clash already (untrained weights).
 // The loop is a serial chain: 20 normalisations of 0.55 us in each step, on one compute unit per clip, 724 us for 32
 // clips of 64 frames and 32 slots.  With the pairs ahead 80 us (steps 1 .. 3 by the loop, 0.8 us for each step after).
 // sig is read while it is written: each word is stored and loaded by itself at device scope, is 0 before this launch
 // and carries TRK_READY, so the loop needs no order between words and never waits.
-constexpr float TRK_MARGIN = 0.1f;
+constexpr float TRK_MARGIN = 0.1f, TRK_CONF_MARGIN = 0.03f;
 constexpr int TRK_EARLY = 5;
 constexpr int TRK_READY = 1 << 30, TRK_FLAT = 1 << 29, TRK_CONF = 1 << 28, TRK_IDX = 0xffff;
 constexpr int TRK_AHEAD = 3;     // first frame matched ahead: by then the loop has run the steps before it
@@ -616,7 +624,7 @@ __device__ __forceinline__ void track_pair(const float* __restrict__ cf, int* __
     bool good = true;
     if (line < N) {
       const float lb = __logf(bv);
-      good = lb - v2 > TRK_MARGIN && fabsf(bv - 0.3f) > 1e-2f && s_cnt[line] <= 1;   // NaN: not good
+      good = lb - v2 > TRK_MARGIN && fabsf(bv - 0.3f) > TRK_CONF_MARGIN && s_cnt[line] <= 1;   // NaN: not good
     }
     if (!__syncthreads_and(good)) return;
   }
@@ -936,6 +944,12 @@ static int track_check(int64_t N, int64_t D, int dtype) {
   return 0;
 }
 
+// Whether the order of a pair's rows moves its values by less than the margins that the pairs matched ahead keep (see
+// track_pair): M = 2 clamp / temperature below 2^19, where fp32's unit is 1/32
+static bool track_order_safe(float inv_t, int64_t n_iters) {
+  return 2.f * TRK_COST_CLAMP * inv_t < 524288.f && n_iters <= 1024;
+}
+
 static float inv_temperature(float temperature) { return 1.f / (temperature > 1e-6f ? temperature : 1e-6f); }
 
 static size_t al256t(size_t v) { return (v + 255) / 256 * 256; }
@@ -1134,7 +1148,9 @@ extern "C" int hclsm_slot_track_sequence(const float* slots, const float* alive,
   //   over 32 slots crowd a compute unit's LDS), hence half as many clips above 32 slots; 3 frames are run by the loop.
   int cus = 0;
   if ((rc = device_cus(&cus))) return rc;
-  const bool ahead = T >= 4 && batch <= (N <= 32 ? cus : cus / 2) && batch * T <= 0x7fffffffLL;
+  const float inv_t = inv_temperature(temperature);
+  const bool ahead = T >= 4 && batch <= (N <= 32 ? cus : cus / 2) && batch * T <= 0x7fffffffLL &&
+                     track_order_safe(inv_t, n_iters);
   int* sig = reinterpret_cast<int*>(ws + L.sig);
   if (T > 1) {
     // pair MLP over every (t-1, t) frame pair: U = W1a s + b1 and V = W1b s for every node row
@@ -1160,7 +1176,6 @@ extern "C" int hclsm_slot_track_sequence(const float* slots, const float* alive,
     a.nt = (int)(T - 1); a.tstride = (int)T; a.fboff = 1;
     if ((rc = launch_cost_dt(dtype, a, st))) return rc;
   }
-  const float inv_t = inv_temperature(temperature);
   rc = with_tile(N, [&](auto cpl) {
     constexpr int CPL = decltype(cpl)::value;
     const unsigned pairs = ahead ? (unsigned)(batch * (T - TRK_AHEAD)) : 0u;

@@ -100,3 +100,20 @@ def test_published_pairs(B, T, N, D, dead, decisive, dup, some):
     done, left = _check(*_run(slots, alive, TrackerWeights.from_module(m, torch.float32)))
     for have, want in ((done, some[0]), (left, some[1])):
         assert want is None or want == (have > 0), (done, left)
+
+
+@pytest.mark.parametrize("temperature,n_iters,beside", [
+    (0.05, 20, True), (0.039, 20, True), (1.0, 20, None), (0.05, 1024, None), (0.038, 20, False), (0.001, 20, False),
+    (0.05, 1025, False)])
+def test_only_where_the_order_of_the_rows_cannot_matter(temperature, n_iters, beside):
+    """The first column step rounds to one unit of 2e4 / temperature.  Where two such units reach the margin of the
+    published matches (0.1 in log units), or rounding can add up over the rounds, the loop does every step."""
+    from hclsm_amd.kernels.slot_tracker import TrackerWeights
+    m = _tracker(64, 32, 8.0, 7)
+    slots, alive = _clips(2, 9, 32, 64, 3, 0.2)
+    W = TrackerWeights.from_module(m, torch.float32)
+    perm, cost, words = _run(slots, alive, W, n_iters, temperature)
+    if beside is not None:
+        assert bool((words & READY).any()) == beside
+    perm2, _, _ = _run(slots.repeat(200, 1, 1, 1), alive.repeat(200, 1, 1), W, n_iters, temperature)   # loops alone
+    assert torch.equal(perm, perm2[:2])
