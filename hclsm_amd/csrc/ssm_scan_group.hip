@@ -9,10 +9,10 @@
 //
 // SG = 16, bf16 I/O: the input term u B_t and its add into h run on the matrix core (v_mfma_f32_32x32x8_bf16; see
 // ssm_scan_fwd_mfma_kernel for the layout).  u = dt x is split exactly into three bf16 pieces (two hold a product of
-// two bf16 values; the clamped dt of the model and block modes has 24 bits), so the products are exact in fp32.  A
-// lane's column also meets the other half's channel with zero weights, so a non-finite u must not enter the operand:
-// the operand takes u clamped to the finite range and the difference (0, +-inf or NaN) is added to the lane's own
-// states instead.  SG = 8: multiply and FMA on the VALU (an fp32 MFMA shares the VALU's multipliers: measured 6.5 ns
+// two bf16 values; the clamped dt of the model and block modes has 24 bits), so the products are exact in fp32.  That
+// holds for finite values only: a lane's column also meets the other half's channel with zero weights, and a zero piece
+// of u meets B.  So from the first chunk on in which any lane's u or any B of the wave's states is not finite, a wave
+// takes its steps on the VALU (a branch inside each step cost 1 to 13%).  SG = 8: multiply and FMA (an fp32 MFMA shares the VALU's multipliers: measured 6.5 ns
 // per 4x4x1 product next to a stream of FMAs, against 1.75 ns per FMA).
 //
 // Bound by VALU issue: 5 issue slots per state update on the matrix core (exponent multiply, exp = 2, decay multiply,
@@ -151,10 +151,8 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
     }
     const float u = dtc * xs;
     if constexpr (MM) {
-      const float uf = __builtin_amdgcn_fmed3f(u, -__FLT_MAX__, __FLT_MAX__);
-      const float e = u - uf;                    // 0 for finite u
-      const uint32_t u1 = __float_as_uint(uf) & 0xffff0000u;
-      const float r1 = uf - __uint_as_float(u1);
+      const uint32_t u1 = __float_as_uint(u) & 0xffff0000u;
+      const float r1 = u - __uint_as_float(u1);
       const uint32_t u2 = __float_as_uint(r1) & 0xffff0000u;
       bop.x = (short)(u1 >> 16);
       bop.y = (short)(u2 >> 16);
@@ -165,7 +163,7 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
         aop.z = (short)bb;
       }
 #pragma unroll
-      for (int s = 0; s < SG; ++s) h[s] = fmaf(h[s], gt[s], e);
+      for (int s = 0; s < SG; ++s) h[s] *= gt[s];
       h = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(aop, bop, h, 0, 0, 0);
     } else {
 #pragma unroll
@@ -202,8 +200,19 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
 
   load(0, xv, dv, bv);
   gates(dv[0]);
-  int buf = 0;
-  for (int t0 = 0; t0 < T; t0 += TC) {
+  int buf = 0, t0 = 0;
+  for (; t0 < T; t0 += TC) {
+    if constexpr (MM) {                          // (past T: the last step's values again)
+      float z = 0.f;                             // NaN if any u is not finite (a clamped dt is)
+      uint32_t b = 0;
+#pragma unroll
+      for (int j = 0; j < TC; ++j) {
+        z = fmaf(MODE == HCLSM_SCAN_RAW ? dv[j] * xv[j] : xv[j], 0.f, z);
+        const uint32_t m = bv[j] & 0x7fffu;
+        b = b > m ? b : m;
+      }
+      if (__any(z != z || b >= 0x7f80u)) break;
+    }
     float xn[TC], dn[TC];
     uint16_t bn[MM ? TC : 1];
     load(t0 + TC, xn, dn, bn);
@@ -229,6 +238,32 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
 #pragma unroll
     for (int j = 0; j < TC; ++j) { xv[j] = xn[j]; dv[j] = dn[j]; if constexpr (MM) bv[j] = bn[j]; }
     buf ^= 1;
+  }
+  if constexpr (MM) {   // from the first chunk with a value that is not finite: this wave's steps on the VALU
+    for (; t0 < T; t0 += TC) {
+#pragma unroll 1
+      for (int j = 0; j < TC && t0 + j < T; ++j) {
+        const int t = t0 + j;
+        const float xs = buf_ld<DT>(rx, vo, t * pitch), d1 = scan_dt<MODE>(buf_ld<DT>(rd, vo, t * pitch)), u = d1 * xs;
+        float yo = 0.f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) { bw[i] = bw0[(size_t)t * rw + i]; cw[i] = cw0[(size_t)t * rw + i]; }
+#pragma unroll
+        for (int s = 0; s < SG; ++s) {
+          h[s] = fmaf(fast_exp2(d1 * a2[s]), h[s], u * word(bw, s));
+          yo = fmaf(h[s], word(cw, s), yo);
+        }
+        red[((buf * TC + j) * NG + g) * 64 + l] = skip ? fmaf(dsk, xs, yo) : yo;
+      }
+      __syncthreads();
+#pragma unroll 1
+      for (int j = g; j < TC && t0 + j < T; j += NG) {
+        float gw = 0.f;
+        if constexpr (MODE == SCAN_BLOCK) gw = buf_ld<DT>(rg, vo, (t0 + j) * pitch);
+        finish(t0 + j, buf * TC + j, gw);
+      }
+      buf ^= 1;
+    }
   }
 
   if (h_final != nullptr && act) {
