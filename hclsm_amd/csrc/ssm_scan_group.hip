@@ -11,9 +11,12 @@
 // ssm_scan_fwd_mfma_kernel for the layout).  u = dt x is split exactly into three bf16 pieces (two hold a product of
 // two bf16 values; the clamped dt of the model and block modes has 24 bits), so the products are exact in fp32.  That
 // holds for finite values only: a lane's column also meets the other half's channel with zero weights, and a zero piece
-// of u meets B.  So from the first chunk on in which any lane's u or any B of the wave's states is not finite, a wave
-// takes its steps on the VALU (a branch inside each step cost 1 to 13%).  SG = 8: multiply and FMA (an fp32 MFMA shares the VALU's multipliers: measured 6.5 ns
-// per 4x4x1 product next to a stream of FMAs, against 1.75 ns per FMA).
+// of u meets B.  So in a chunk with a u or a B of the wave's states that is not finite, the products with such a value
+// are formed on the VALU and the operands have 0 there; what is finite comes out the same.  (One test per chunk and a
+// scalar branch per step, 89 registers, five waves per SIMD; clamping u in every step took 96 to 101 registers, 1024 x 64
+// x 384, S 32, model 167 against 153 us.  A second loop for such chunks took 108 to 128 registers: 161 to 200.)
+// SG = 8: multiply and FMA on the VALU (an fp32 MFMA shares the VALU's multipliers: measured 6.5 ns per 4x4x1 product
+// next to a stream of FMAs, against 1.75 ns per FMA).
 //
 // Bound by VALU issue: 5 issue slots per state update on the matrix core (exponent multiply, exp = 2, decay multiply,
 // readout FMA), 6 on the VALU.  Measured on MI355X (us per launch; before: one to four lanes per channel, states
@@ -45,7 +48,7 @@ __device__ __forceinline__ float exp_comp(float v) {
 }
 
 template <int DT, int MODE, int SG, int TC>
-__global__ void __launch_bounds__(64 * GRP_MAX_WAVES)
+__global__ void __launch_bounds__(64 * GRP_MAX_WAVES) __attribute__((amdgpu_waves_per_eu(SG == 16 ? 5 : 4)))
 ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const typename Elem<DT>::T* __restrict__ dt,
                           const float* __restrict__ A_log, const typename Elem<DT>::T* __restrict__ Bm,
                           const typename Elem<DT>::T* __restrict__ Cm, const float* __restrict__ Dskip,
@@ -141,7 +144,7 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
     if constexpr (DT == HCLSM_BF16) return __uint_as_float(s & 1 ? w[s >> 1] & 0xffff0000u : w[s >> 1] << 16);
     else return __uint_as_float(w[s]);
   };
-  auto step = [&](int t, int slot, float xs, float dnext, uint16_t bb) {
+  auto step = [&](bool odd, int t, int slot, float xs, float dnext, uint16_t bb) {
     const int tn = t + 1 < T ? t + 1 : T - 1;
     uint32_t cwn[NW], bwn[NW];
 #pragma unroll
@@ -149,8 +152,20 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
       cwn[i] = cw0[(size_t)tn * rw + i];
       if constexpr (!MM) bwn[i] = bw0[(size_t)tn * rw + i];
     }
-    const float u = dtc * xs;
+    float u = dtc * xs;
     if constexpr (MM) {
+#pragma unroll
+      for (int s = 0; s < SG; ++s) h[s] *= gt[s];
+      if (__builtin_expect(odd, 0)) {            // products with a value that is not finite
+        const bool uf = fabsf(u) <= __FLT_MAX__;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) bw[i] = bw0[(size_t)t * rw + i];
+#pragma unroll
+        for (int s = 0; s < SG; ++s)
+          if (!(uf && fabsf(word(bw, s)) <= __FLT_MAX__)) h[s] = fmaf(u, word(bw, s), h[s]);
+        u = uf ? u : 0.f;
+        bb = (bb & 0x7f80) == 0x7f80 ? 0 : bb;
+      }
       const uint32_t u1 = __float_as_uint(u) & 0xffff0000u;
       const float r1 = u - __uint_as_float(u1);
       const uint32_t u2 = __float_as_uint(r1) & 0xffff0000u;
@@ -162,8 +177,6 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
         bop.z = (short)(__float_as_uint(r2) >> 16);
         aop.z = (short)bb;
       }
-#pragma unroll
-      for (int s = 0; s < SG; ++s) h[s] *= gt[s];
       h = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(aop, bop, h, 0, 0, 0);
     } else {
 #pragma unroll
@@ -200,10 +213,11 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
 
   load(0, xv, dv, bv);
   gates(dv[0]);
-  int buf = 0, t0 = 0;
-  for (; t0 < T; t0 += TC) {
+  int buf = 0;
+  for (int t0 = 0; t0 < T; t0 += TC) {
+    bool odd = false;                            // the chunk has a u or a B that is not finite
     if constexpr (MM) {                          // (past T: the last step's values again)
-      float z = 0.f;                             // NaN if any u is not finite (a clamped dt is)
+      float z = 0.f;                             // NaN if any u is not finite (a clamped dt always is)
       uint32_t b = 0;
 #pragma unroll
       for (int j = 0; j < TC; ++j) {
@@ -211,7 +225,7 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
         const uint32_t m = bv[j] & 0x7fffu;
         b = b > m ? b : m;
       }
-      if (__any(z != z || b >= 0x7f80u)) break;
+      odd = __any(z != z || b >= 0x7f80u);
     }
     float xn[TC], dn[TC];
     uint16_t bn[MM ? TC : 1];
@@ -227,7 +241,7 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
     }
 #pragma unroll
     for (int j = 0; j < TC; ++j)
-      if (t0 + j < T) step(t0 + j, buf * TC + j, xv[j], j + 1 < TC ? dv[j + 1 < TC ? j + 1 : 0] : dn[0],
+      if (t0 + j < T) step(odd, t0 + j, buf * TC + j, xv[j], j + 1 < TC ? dv[j + 1 < TC ? j + 1 : 0] : dn[0],
                            bv[MM ? j : 0]);
     __syncthreads();
 #pragma unroll
@@ -238,32 +252,6 @@ ssm_scan_fwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
 #pragma unroll
     for (int j = 0; j < TC; ++j) { xv[j] = xn[j]; dv[j] = dn[j]; if constexpr (MM) bv[j] = bn[j]; }
     buf ^= 1;
-  }
-  if constexpr (MM) {   // from the first chunk with a value that is not finite: this wave's steps on the VALU
-    for (; t0 < T; t0 += TC) {
-#pragma unroll 1
-      for (int j = 0; j < TC && t0 + j < T; ++j) {
-        const int t = t0 + j;
-        const float xs = buf_ld<DT>(rx, vo, t * pitch), d1 = scan_dt<MODE>(buf_ld<DT>(rd, vo, t * pitch)), u = d1 * xs;
-        float yo = 0.f;
-#pragma unroll
-        for (int i = 0; i < NW; ++i) { bw[i] = bw0[(size_t)t * rw + i]; cw[i] = cw0[(size_t)t * rw + i]; }
-#pragma unroll
-        for (int s = 0; s < SG; ++s) {
-          h[s] = fmaf(fast_exp2(d1 * a2[s]), h[s], u * word(bw, s));
-          yo = fmaf(h[s], word(cw, s), yo);
-        }
-        red[((buf * TC + j) * NG + g) * 64 + l] = skip ? fmaf(dsk, xs, yo) : yo;
-      }
-      __syncthreads();
-#pragma unroll 1
-      for (int j = g; j < TC && t0 + j < T; j += NG) {
-        float gw = 0.f;
-        if constexpr (MODE == SCAN_BLOCK) gw = buf_ld<DT>(rg, vo, (t0 + j) * pitch);
-        finish(t0 + j, buf * TC + j, gw);
-      }
-      buf ^= 1;
-    }
   }
 
   if (h_final != nullptr && act) {
