@@ -51,6 +51,7 @@ __device__ __forceinline__ void split_op(float v, s16x4_t& o) {
     if constexpr (NP >= 3) o.z = (short)(__float_as_uint(r1 - __uint_as_float(p2)) >> 16);
   }
 }
+__device__ __forceinline__ bool finite_f(float v) { return fabsf(v) <= __FLT_MAX__; }
 __device__ __forceinline__ s16x4_t fill_op(uint16_t b, int np) {
   return s16x4_t{(short)b, (short)(np >= 2 ? b : 0), (short)(np >= 3 ? b : 0), 0};
 }
@@ -88,6 +89,7 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
   float* sG = sU + BG_WIN * 64;                  //   and the gradient of the scan output (0 there)
   uint16_t* sBh = reinterpret_cast<uint16_t*>(sG + BG_WIN * 64);   // [BG_WIN][SH], matrix core
   uint16_t* sCh = sBh + BG_WIN * SH;
+  int* sOdd = reinterpret_cast<int*>(sCh + BG_WIN * SH);           // matrix core: a staged value is not finite
 
   const int s0 = g * SG;
   const int d = blockIdx.y * 64 + l;
@@ -104,9 +106,25 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
     a2[j] = -((MODE != HCLSM_SCAN_RAW) ? fminf(fmaxf(e, 1e-6f), 1.0f) : e) * HCLSM_LOG2E;
   }
   const float dsk = Dskip ? Dskip[dd] : 0.f;
+  if (MM && threadIdx.x == 0) *sOdd = 0;
   if constexpr (MM)
     for (int e = threadIdx.x; e < 2 * BG_WIN * 2; e += blockDim.x) (e & 1 ? sCh : sBh)[(e >> 2) * SH + S + ((e >> 1) & 1)] = 0;
 
+  // The matrix core takes finite values only: a lane's column also meets the other half's channel with zero weights, and a
+  // zero piece of u meets B.  From the first window with a value that is not finite on, `odd` is set and the products
+  // with such a value are formed here instead (v: u or gy, w: the row's B or C), in the states' place; the operands have
+  // 0 there.  What is finite comes out the same either way.
+  bool odd = false;
+  auto fix_up = [&](f32x16_t& st, float& v, uint16_t& w_op, const uint16_t* w) {
+    const bool vf = finite_f(v);
+#pragma unroll
+    for (int j = 0; j < SG; ++j) {
+      const float wj = bf16_bits_to_f32(w[j]);
+      if (!(vf && finite_f(wj))) st[j] = fmaf(v, wj, st[j]);
+    }
+    v = vf ? v : 0.f;
+    w_op = (w_op & 0x7f80) == 0x7f80 ? 0 : w_op;
+  };
   f32x16_t gh;
   float gA[SG], gD = 0.f;
 #pragma unroll
@@ -127,6 +145,13 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
     const auto rgg = rsrc(GATE ? reinterpret_cast<TT*>(gate.g_gate) + row0 * Dn : gx + row0 * Dn, GATE ? slab : 0);
 
     // the rows of window w; steps past T read as zero
+    bool seen = false;                           // this thread staged a value that is not finite (matrix core)
+    auto look = [&](float v) { if constexpr (MM) seen |= !finite_f(v); };
+    auto staged = [&]() {
+      if (MM && seen) *sOdd = 1;
+      __syncthreads();
+      if constexpr (MM) odd = __builtin_amdgcn_readfirstlane(*sOdd);
+    };
     auto stage = [&](int w) {
       for (int e = threadIdx.x; e < BG_WIN * S; e += blockDim.x) {
         const int off = (w * BG_WIN * S + e) * ES;
@@ -135,6 +160,8 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
           const uint16_t c = __builtin_amdgcn_raw_buffer_load_b16(rc, off, 0, 0);
           const int r = e / S;
           sB[e] = bf16_bits_to_f32(b);
+          look(sB[e]);
+          look(bf16_bits_to_f32(c));
           sBh[r * SH + e - r * S] = b;
           sCh[r * SH + e - r * S] = c;
         } else {
@@ -169,8 +196,14 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
           if (r < BG_WIN) {
             const float v = dt_of(dv[k], w * BG_WIN + r < T);
             sDt[r * 64 + l] = v;
-            sU[r * 64 + l] = act ? v * xv[k] : 0.f;
-            if (with_g) sG[r * 64 + l] = act ? (GATE ? gv[k] * silu_f(gt[k]) : gv[k]) : 0.f;
+            const float u = act ? v * xv[k] : 0.f;
+            sU[r * 64 + l] = u;
+            look(u);
+            if (with_g) {
+              const float gr = act ? (GATE ? gv[k] * silu_f(gt[k]) : gv[k]) : 0.f;
+              sG[r * 64 + l] = gr;
+              look(gr);
+            }
           }
         }
       }
@@ -179,16 +212,13 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
     // one forward step: hc = exp(dt A) hc + u B_r (r: row of the window)
     auto fwd_step = [&](int r, float dtv, float u) {
       if constexpr (MM) {
-        // the operand stays finite (its column also meets the other half's channel with zero weights); what is not
-        // is added to the lane's own states
-        const float uf = __builtin_amdgcn_fmed3f(u, -__FLT_MAX__, __FLT_MAX__);
-        const float e = u - uf;
-        s16x4_t bop = {0, 0, 0, 0};
-        split_op<NPU>(uf, bop);
-        const s16x4_t aop = fill_op(sBh[r * SH + op_col], NPU);
+        uint16_t b = sBh[r * SH + op_col];
 #pragma unroll
-        for (int j = 0; j < SG; ++j) hc[j] = fmaf(fast_exp2(dtv * a2[j]), hc[j], e);
-        hc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(aop, bop, hc, 0, 0, 0);
+        for (int j = 0; j < SG; ++j) hc[j] *= fast_exp2(dtv * a2[j]);
+        if (__builtin_expect(odd, 0)) fix_up(hc, u, b, sBh + r * SH + s0);
+        s16x4_t bop = {0, 0, 0, 0};
+        split_op<NPU>(u, bop);
+        hc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(fill_op(b, NPU), bop, hc, 0, 0, 0);
       } else {
 #pragma unroll
         for (int j = 0; j < SG; ++j) hc[j] = fmaf(fast_exp2(dtv * a2[j]), hc[j], u * sB[r * S + s0 + j]);
@@ -220,7 +250,7 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
         __syncthreads();
         stage(w);
         stage_values(w, false);
-        __syncthreads();
+        staged();
         sweep(BG_WIN / K, false);
         if (act)
 #pragma unroll
@@ -234,7 +264,7 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
       __syncthreads();
       stage(w);
       stage_values(w, true);
-      __syncthreads();
+      staged();
       const int left = T - w * BG_WIN;
       const int nch = left >= BG_WIN ? BG_WIN / K : (left + K - 1) / K;
       for (int c = nch - 1; c >= 0; --c) {
@@ -274,15 +304,11 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
           const float dv = sDt[r * 64 + l], um = sU[r * 64 + l], gv = sG[r * 64 + l];
           if constexpr (MM) {
             float gf = gv;
-            if (__any(!(fabsf(gf) <= __FLT_MAX__))) {   // as in fwd_step; rare
-              gf = __builtin_amdgcn_fmed3f(gf, -__FLT_MAX__, __FLT_MAX__);
-              const float e = gv - gf;
-#pragma unroll
-              for (int j = 0; j < SG; ++j) gh[j] += e;
-            }
+            uint16_t c_op = sCh[r * SH + op_col];
+            if (__builtin_expect(odd, 0)) fix_up(gh, gf, c_op, sCh + r * SH + s0);
             s16x4_t bop = {0, 0, 0, 0};
             split_op<NPG>(gf, bop);
-            gh = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(fill_op(sCh[r * SH + op_col], NPG), bop, gh, 0, 0, 0);
+            gh = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(fill_op(c_op, NPG), bop, gh, 0, 0, 0);
           }
           float v[SG], q = 0.f, gda2 = 0.f;     // gda2 = sum garg * A * log2(e); times ln 2 below
 #pragma unroll
@@ -368,7 +394,7 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
 
 static size_t group_lds(int NG, int SG, int S, bool mm) {
   size_t f = (size_t)NG * 2 * SG * 64 + (size_t)BG_WIN * S * (mm ? 1 : 2) + (size_t)BG_K * 2 * S + (size_t)BG_K * 2 * NG * 64 + (size_t)3 * BG_WIN * 64;
-  return f * 4 + (mm ? (size_t)2 * BG_WIN * (S + 2) * 2 : 0);
+  return f * 4 + (mm ? (size_t)2 * BG_WIN * (S + 2) * 2 + 4 : 0);
 }
 
 // Sequences one workgroup walks: the fewest rounds of resident workgroups times their length, half a sequence added

@@ -81,3 +81,39 @@ def test_block_forward(dtype):
         y = run(slice(None))
         for n in (0, 1, N - 2, N - 1):
             _same(y[n:n + 1], run(slice(n, n + 1)), 4e-3, n)
+
+
+@pytest.mark.parametrize("which", ["x", "gy", "B", "C"])
+@pytest.mark.parametrize("N,T,Dn,S", [(1100, 9, 64, 48), (1100, 18, 64, 48), (300, 7, 129, 96)])
+@pytest.mark.parametrize("mode", ["raw", "model"])
+def test_backward(N, T, Dn, S, mode, which):
+    """16 states a lane (wide grids) against the same sequences on a grid too small for it (8 a lane; past 64 states the
+    fp32 kernel on the same values)."""
+    from hclsm_amd import _lib
+    from hclsm_amd.kernels.ssm_scan_bwd import scan_backward
+    from hclsm_amd.workloads import scan_inputs
+    d = scan_inputs(N, T, Dn, S, dtype=torch.bfloat16, seed=N + S)
+    if mode == "model":
+        d["A_log"] = -d["A_log"]
+    d["gy"] = torch.randn(N, T, Dn, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+    d["B"][:, :, 3] = 0
+    d["C"][:, :, 4] = 0
+    rows = [0, 1, N // 2, N - 1]
+    for n, bad in zip(rows, (INF, -INF, NAN, INF)):
+        d[which][n, T // 2 if n else T - 1, (5 + 40 * (n & 1)) % S] = bad
+    code = _lib.SCAN_RAW if mode == "raw" else _lib.SCAN_MODEL
+
+    def run(pick, dtype):
+        v = [d[k][pick].cuda().to(dtype) for k in ("x", "dt", "B", "C", "gy")]
+        return scan_backward(v[0], v[1], d["A_log"].cuda(), v[2], v[3], None, v[4], code)
+
+    got = run(slice(None), torch.bfloat16)
+    for n in rows + [2]:
+        ref = run(slice(n, n + 1), torch.bfloat16 if S <= 64 else torch.float32)
+        for k in ("x", "dt", "B", "C"):
+            _same(got[k][n:n + 1], ref[k], 4e-3, (k, n))
+    # gA_log: not finite where any sequence's is
+    odd = torch.zeros_like(got["A_log"], dtype=torch.bool)
+    for n in rows:
+        odd |= ~torch.isfinite(run(slice(n, n + 1), torch.float32)["A_log"])
+    assert torch.equal(~torch.isfinite(got["A_log"]), odd)
