@@ -65,6 +65,13 @@ def block_params(m, x):
     return ps
 
 
+def _aligned(t, n: int = 16):
+    """t contiguous at a multiple of n bytes: t itself, or a copy (torch allocates at 512).  Gradients and unpacked saved
+    tensors may be contiguous views at any offset, where the forward's inputs were checked."""
+    t = t.contiguous()
+    return t if t.data_ptr() % n == 0 else t.clone()
+
+
 def _save_buffer(x, ps, train: bool):
     N, T, d = x.shape
     nb = int(_lib.lib().hclsm_ssm_block_save(N, T, d, ps[8].shape[0], ps[8].shape[1], int(train)))
@@ -92,9 +99,10 @@ class _Block(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, g):
         x, save, *ps = ctx.saved_tensors
+        x, save, ps = _aligned(x), _aligned(save, 256), [_aligned(p) for p in ps]
         N, T, d = x.shape
         di, S = ps[8].shape
-        g = g.to(torch.float32).contiguous()
+        g = _aligned(g.to(torch.float32))
         L = _lib.lib()
         scratch = torch.empty(int(L.hclsm_ssm_block_scratch(N, T, d, di, S)), dtype=torch.uint8, device=x.device)
         gx = torch.empty_like(x)

@@ -1,0 +1,58 @@
+"""The fused Level-0 block inside a larger autograd graph: incoming gradients and saved tensors at any address."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_ssm_block_gpu import _block
+
+pytestmark = pytest.mark.gpu
+
+
+def _grads(m, x, loss):
+    m.zero_grad()
+    x.grad = None
+    loss.backward()
+    return [x.grad.clone()] + [p.grad.clone() for p in m.parameters()]
+
+
+def _run(m, x):
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = m(x)
+    assert type(y.grad_fn).__name__ == "_BlockBackward"
+    return y
+
+
+@pytest.mark.parametrize("S", [16, 48])
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_gradient_at_an_odd_address(S, shift):
+    """The backward of a cat hands a contiguous view at any multiple of 4 bytes over."""
+    m = _block(64, S, 1)
+    x = torch.randn(3, 9, 64, device="cuda").requires_grad_()
+    aux = torch.randn(shift, device="cuda").requires_grad_()
+    w = torch.randn(shift + x.numel(), device="cuda")
+    assert w[shift:].data_ptr() % 16
+    got = _grads(m, x, (torch.cat([aux, _run(m, x).reshape(-1)]) * w).sum())
+    ref = _grads(m, x, (_run(m, x).reshape(-1) * w[shift:].clone()).sum())
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+
+
+def test_saved_tensors_at_an_odd_address():
+    """Saved-tensor hooks that hand back copies inside a larger buffer, one element past its start."""
+    m = _block(64, 32, 2)
+    x = torch.randn(2, 7, 64, device="cuda").requires_grad_()
+    g = torch.randn_like(x)
+
+    def pack(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        buf[1:].copy_(t.detach().reshape(-1))
+        return buf, t.shape
+
+    ref = _grads(m, x, (_run(m, x) * g).sum())
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda h: h[0][1:].view(h[1])):
+        y = _run(m, x)
+    got = _grads(m, x, (y * g).sum())
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
