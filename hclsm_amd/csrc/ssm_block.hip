@@ -448,7 +448,8 @@ static int blk_layout(int64_t N, int64_t T, int64_t d, int64_t di, int64_t S, bo
   L->wt = take(train ? nw * 2 : 0);
   const int64_t scan_ws = hclsm_ssm_scan_bwd_workspace(N, T, di, S);
   if (scan_ws < 0) return (int)scan_ws;
-  L->ck = take(train && L->pair16 ? scan_ws : 0);
+  const int64_t ck_bytes = L->pair16 ? scan_bwd_ck_bytes(N, T, di, S) : 0;   // the forward leaves the scan's checkpoints
+  L->ck = take(train ? ck_bytes : 0);
   L->save = o;
   o = 0;
   L->gy = take(R * di * 2); L->gys = take(L->group ? 0 : R * di * 2); L->gz0 = take(R * di * 2); L->gdt = take(R * di * 2);
@@ -463,19 +464,21 @@ static int blk_layout(int64_t N, int64_t T, int64_t d, int64_t di, int64_t S, bo
   L->part = take((size_t)L->splits * L->part_ld * 4);
   L->ln_blocks = (int)((R + 15) / 16 < 256 ? (R + 15) / 16 : 256);
   L->lnp = take((size_t)L->ln_blocks * 2 * d * 4);
-  L->scan = take(L->pair16 ? 0 : scan_ws);
+  L->scan = take(scan_ws - ck_bytes);
   L->scratch = o;
   return 0;
 }
 
+template <typename U>
 struct BlkW {   // 16-bit weights and their transposes inside the save buffer
-  uint16_t *in, *gate, *dt, *b, *c, *out, *in_t, *gate_t, *dt_t, *bc_t, *out_t;
+  U *in, *gate, *dt, *b, *c, *out, *in_t, *gate_t, *dt_t, *bc_t, *out_t;
 };
-static BlkW blk_weights(char* save, const BlkLayout& L, int64_t d, int64_t di, int64_t S) {
-  BlkW w;
-  uint16_t* p = reinterpret_cast<uint16_t*>(save + L.w);
+template <typename U, typename Byte>
+static BlkW<U> blk_weights(Byte* save, const BlkLayout& L, int64_t d, int64_t di, int64_t S) {
+  BlkW<U> w;
+  U* p = reinterpret_cast<U*>(save + L.w);
   w.in = p; p += di * d; w.gate = p; p += di * d; w.dt = p; p += di * di; w.b = p; p += S * di; w.c = p; p += S * di; w.out = p;
-  p = reinterpret_cast<uint16_t*>(save + L.wt);
+  p = reinterpret_cast<U*>(save + L.wt);
   w.in_t = p; p += di * d; w.gate_t = p; p += di * d; w.dt_t = p; p += di * di; w.bc_t = p; p += 2 * S * di; w.out_t = p;
   return w;
 }
@@ -536,7 +539,7 @@ extern "C" int hclsm_ssm_block_forward(const HclsmBlockParams* P, const float* x
   if (((uintptr_t)save & 255) != 0) return HCLSM_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
   char* s = reinterpret_cast<char*>(save);
-  const BlkW w = blk_weights(s, L, d, di, S);
+  const BlkW<uint16_t> w = blk_weights<uint16_t>(s, L, d, di, S);
   CastJobs js = {};
   auto job = [&](const float* src, uint16_t* dst, uint16_t* dst_t, int64_t rows, int64_t cols, int64_t ld_t) {
     const int b0 = js.n ? js.j[js.n - 1].blk0 + ((js.j[js.n - 1].rows + 31) / 32) * ((js.j[js.n - 1].cols + 31) / 32) : 0;
@@ -572,8 +575,8 @@ extern "C" int hclsm_ssm_block_forward(const HclsmBlockParams* P, const float* x
   if ((rc = run_gemm(g, L.R, st))) return rc;
   void* y_pre = train ? s + L.y_pre : nullptr;
   if (train && L.pair16)
-    rc = hclsm_ssm_block_scan_fwd_ckpt(s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, s + L.gate, s + L.y, y_pre, nullptr,
-                                       batch, T, di, S, HCLSM_BF16, s + L.ck, (int64_t)(L.save - L.ck), stream);
+    rc = scan_fwd_ckpt(SCAN_BLOCK, s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, nullptr, s + L.y, nullptr, batch, T, di,
+                       S, HCLSM_BF16, s + L.gate, y_pre, reinterpret_cast<float*>(s + L.ck), st);
   else
     rc = hclsm_ssm_block_scan_fwd(s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, s + L.gate, s + L.y, y_pre, nullptr,
                                   batch, T, di, S, HCLSM_BF16, stream);
@@ -600,9 +603,9 @@ extern "C" int hclsm_ssm_block_backward(const HclsmBlockParams* P, const float* 
   if (save_bytes < (int64_t)L.save || scratch_bytes < (int64_t)L.scratch) return HCLSM_ERR_SHAPE;
   if (((uintptr_t)save & 255) || ((uintptr_t)scratch & 255) || !al16p(g)) return HCLSM_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  char* s = reinterpret_cast<char*>(const_cast<void*>(save));
+  const char* s = reinterpret_cast<const char*>(save);
   char* q = reinterpret_cast<char*>(scratch);
-  const BlkW w = blk_weights(s, L, d, di, S);
+  const BlkW<const uint16_t> w = blk_weights<const uint16_t>(s, L, d, di, S);
   uint16_t* gB = reinterpret_cast<uint16_t*>(q + L.gbc);
   uint16_t* gC = reinterpret_cast<uint16_t*>(q + L.gbc + up256(L.R * S * 2));
   GemmGroup gg = {};
@@ -614,7 +617,7 @@ extern "C" int hclsm_ssm_block_backward(const HclsmBlockParams* P, const float* 
     BwdGate gate;
     gate.gate = s + L.gate; gate.y_pre = s + L.y_pre; gate.g_gate = q + L.gg;
     rc = scan_bwd_block(s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, q + L.gy, q + L.gz0, q + L.gdt, G->a_log, gB, gC,
-                        batch, T, di, S, HCLSM_BF16, gate, q + L.scan, (int64_t)(L.scratch - L.scan), false, st);
+                        batch, T, di, S, HCLSM_BF16, gate, nullptr, q + L.scan, (int64_t)(L.scratch - L.scan), st);
   } else {
     const int64_t n2 = L.R * di / 2;
     const int64_t nb = (n2 + 255) / 256;
@@ -623,7 +626,8 @@ extern "C" int hclsm_ssm_block_backward(const HclsmBlockParams* P, const float* 
                        (uint32_t*)(q + L.gys), (uint32_t*)(q + L.gg), n2);
     HCLSM_LAUNCH_CHECK();
     rc = scan_bwd_block(s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, q + L.gys, q + L.gz0, q + L.gdt, G->a_log, gB, gC,
-                        batch, T, di, S, HCLSM_BF16, BwdGate(), s + L.ck, (int64_t)(L.save - L.ck), true, st);
+                        batch, T, di, S, HCLSM_BF16, BwdGate(), reinterpret_cast<const float*>(s + L.ck), q + L.scan,
+                        (int64_t)(L.scratch - L.scan), st);
   }
   if (rc) return rc;
   gg = {};

@@ -422,7 +422,7 @@ static int launch_tail(const float* ga, const float* gd, const float* gbc, const
 template <int DT, int SP, int MODE>
 static int launch_bwd(const void* x, const void* dt, const float* A_log, const void* B, const void* C,
                       const float* Dskip, const void* gy, void* gx, void* gdt, float* gA_log, void* gB, void* gC,
-                      float* gD, char* ws, const BwdWs& L, int64_t N, int64_t T, int64_t Dn, int64_t S,
+                      float* gD, char* ws, float* ck, const BwdWs& L, int64_t N, int64_t T, int64_t Dn, int64_t S,
                       bool have_ck, hipStream_t st) {
   using TT = typename Elem<DT>::T;
   constexpr int SG = bwd_sg(SP);
@@ -437,7 +437,7 @@ static int launch_bwd(const void* x, const void* dt, const float* A_log, const v
   float* gbc = reinterpret_cast<float*>(ws + L.gbc);
   hipLaunchKernelGGL((ssm_scan_bwd_kernel<DT, SP, MODE>), dim3((unsigned)N, (unsigned)nblk_d), dim3(threads), 0, st,
                      (const TT*)x, (const TT*)dt, A_log, (const TT*)B, (const TT*)C, Dskip, (const TT*)gy, (TT*)gx,
-                     (TT*)gdt, reinterpret_cast<float*>(ws + L.ck), gbc, reinterpret_cast<float*>(ws + L.ga),
+                     (TT*)gdt, ck, gbc, reinterpret_cast<float*>(ws + L.ga),
                      reinterpret_cast<float*>(ws + L.gd), a);
   HCLSM_LAUNCH_CHECK();
   return launch_tail<DT, MODE>(reinterpret_cast<const float*>(ws + L.ga), reinterpret_cast<const float*>(ws + L.gd),
@@ -457,7 +457,7 @@ static int scan_bwd_entry(const void* x, const void* dt, const float* A_log, con
                           const float* Dskip, const void* gy, void* gx, void* gdt, float* gA_log, void* gB, void* gC,
                           float* gD, int64_t batch, int64_t T, int64_t d_inner, int64_t d_state, int dtype, int mode,
                           void* workspace, int64_t workspace_bytes, bool have_ck, void* stream,
-                          BwdGate gate = BwdGate()) {
+                          BwdGate gate = BwdGate(), const float* ck_in = nullptr) {
   if (batch < 0 || T < 0 || d_inner < 0 || d_state < 1) return HCLSM_ERR_SHAPE;
   if (batch > 0x7fffffffLL || T > 0x7fffffffLL || d_inner > 0x7fffffffLL) return HCLSM_ERR_SHAPE;
   if (d_state > 128) return HCLSM_ERR_UNSUPPORTED;
@@ -477,16 +477,22 @@ static int scan_bwd_entry(const void* x, const void* dt, const float* A_log, con
   }
   if (!x || !dt || !A_log || !B || !C || !gy || !gx || !gdt || !gA_log || !gB || !gC || !workspace)
     return HCLSM_ERR_NULL;
-  const BwdWs L = bwd_ws(batch, T, d_inner, d_state);
+  BwdWs L = bwd_ws(batch, T, d_inner, d_state);
+  if (ck_in) {   // the checkpoints are elsewhere: the workspace has the partial sums only
+    const size_t skip = L.gbc;
+    L.gbc -= skip; L.ga -= skip; L.gd -= skip; L.total -= skip;
+  }
   if (workspace_bytes < (int64_t)L.total) return HCLSM_ERR_SHAPE;
   char* ws = reinterpret_cast<char*>(workspace);
+  // (the kernel writes its checkpoints only where it has none)
+  float* ck = ck_in ? const_cast<float*>(ck_in) : reinterpret_cast<float*>(ws + L.ck);
   if (!have_ck && bwd_group_ok(T, d_inner, d_state, dtype)) {
     // wide states: their groups over the waves of a workgroup (its partials fit the regions of the layout above)
     float* gbc = reinterpret_cast<float*>(ws + L.gbc);
     float *ga = reinterpret_cast<float*>(ws + L.ga), *gd = reinterpret_cast<float*>(ws + L.gd);
     int parts = 0;
     const int rc = bwd_group(gate.gate ? BWD_BLOCK_GATE : mode, x, dt, A_log, B, C, Dskip, gy, gx, gdt, gate,
-                             reinterpret_cast<float*>(ws + L.ck), gbc, ga, gd, batch, T, d_inner, d_state, dtype, &parts,
+                             ck, gbc, ga, gd, batch, T, d_inner, d_state, dtype, &parts,
                              st);
     if (rc) return rc;
     const int nblk = (int)((d_inner + 63) / 64);
@@ -504,12 +510,12 @@ static int scan_bwd_entry(const void* x, const void* dt, const float* A_log, con
 #define HCLSM_BWD(DT_, SP_)                                                                                  \
   if (sp_of(d_state) == SP_) {                                                                               \
     if (mode == HCLSM_SCAN_RAW)                                                                              \
-      return launch_bwd<DT_, SP_, HCLSM_SCAN_RAW>(x, dt, A_log, B, C, Dskip, gy, gx, gdt, gA_log, gB, gC, gD, ws, L, \
+      return launch_bwd<DT_, SP_, HCLSM_SCAN_RAW>(x, dt, A_log, B, C, Dskip, gy, gx, gdt, gA_log, gB, gC, gD, ws, ck, L, \
                                                   batch, T, d_inner, d_state, have_ck, st);                  \
     if (mode == HCLSM_SCAN_BLOCK)                                                                            \
       return launch_bwd<DT_, SP_, HCLSM_SCAN_BLOCK>(x, dt, A_log, B, C, Dskip, gy, gx, gdt, gA_log, gB, gC, gD, ws, \
-                                                    L, batch, T, d_inner, d_state, have_ck, st);             \
-    return launch_bwd<DT_, SP_, HCLSM_SCAN_MODEL>(x, dt, A_log, B, C, Dskip, gy, gx, gdt, gA_log, gB, gC, gD, ws, L, \
+                                                    ck, L, batch, T, d_inner, d_state, have_ck, st);             \
+    return launch_bwd<DT_, SP_, HCLSM_SCAN_MODEL>(x, dt, A_log, B, C, Dskip, gy, gx, gdt, gA_log, gB, gC, gD, ws, ck, L, \
                                                   batch, T, d_inner, d_state, have_ck, st);                  \
   }
 #define HCLSM_BWD_DT(DT_) \
@@ -524,10 +530,13 @@ static int scan_bwd_entry(const void* x, const void* dt, const float* A_log, con
 
 int hclsm::scan_bwd_block(const void* z, const void* dt_in, const float* A_log, const void* B, const void* C,
                           const void* gy, void* gz, void* gdt, float* gA_log, void* gB, void* gC, int64_t batch, int64_t T,
-                          int64_t d_inner, int64_t d_state, int dtype, BwdGate gate, void* ws, int64_t ws_bytes,
-                          bool have_ck, hipStream_t st) {
+                          int64_t d_inner, int64_t d_state, int dtype, BwdGate gate, const float* ck, void* ws,
+                          int64_t ws_bytes, hipStream_t st) {
   return scan_bwd_entry(z, dt_in, A_log, B, C, nullptr, gy, gz, gdt, gA_log, gB, gC, nullptr, batch, T, d_inner, d_state,
-                        dtype, HCLSM_SCAN_BLOCK, ws, ws_bytes, have_ck, (void*)st, gate);
+                        dtype, HCLSM_SCAN_BLOCK, ws, ws_bytes, ck != nullptr, (void*)st, gate, ck);
+}
+int64_t hclsm::scan_bwd_ck_bytes(int64_t batch, int64_t T, int64_t d_inner, int64_t d_state) {
+  return (int64_t)bwd_ws(batch, T, d_inner, d_state).gbc;
 }
 
 extern "C" int hclsm_ssm_scan_bwd(const void* x, const void* dt, const float* A_log, const void* B, const void* C,

@@ -23,9 +23,11 @@ int bwd_group(int mode, const void* x, const void* dt, const float* A_log, const
               float* gd, int64_t N, int64_t T, int64_t Dn, int64_t S, int dtype, int* parts, hipStream_t st);
 
 // The block-mode backward as composite entry points call it (ssm_scan_bwd.hip): with gate set, gy is the gradient of the
-// gated output (shapes of bwd_group_ok); with have_ck the workspace holds the checkpointing forward's states.
+// gated output (shapes of bwd_group_ok).  ck (nullable): the checkpointing forward's states, scan_bwd_ck_bytes of them, only
+// read; ws then holds the partial sums alone, hclsm_ssm_scan_bwd_workspace - scan_bwd_ck_bytes.
+int64_t scan_bwd_ck_bytes(int64_t batch, int64_t T, int64_t d_inner, int64_t d_state);
 int scan_bwd_block(const void* z, const void* dt_in, const float* A_log, const void* B, const void* C, const void* gy,
                    void* gz, void* gdt, float* gA_log, void* gB, void* gC, int64_t batch, int64_t T, int64_t d_inner,
-                   int64_t d_state, int dtype, BwdGate gate, void* ws, int64_t ws_bytes, bool have_ck, hipStream_t st);
+                   int64_t d_state, int dtype, BwdGate gate, const float* ck, void* ws, int64_t ws_bytes, hipStream_t st);
 
 }  // namespace hclsm

@@ -1,4 +1,5 @@
-"""The fused Level-0 block inside a larger autograd graph: incoming gradients and saved tensors at any address."""
+"""The fused Level-0 block inside a larger autograd graph: incoming gradients and saved tensors at any address, the saved
+forward left as it is."""
 
 from __future__ import annotations
 
@@ -55,4 +56,21 @@ def test_saved_tensors_at_an_odd_address():
         y = _run(m, x)
     got = _grads(m, x, (y * g).sum())
     for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("S", [16, 48])
+def test_the_backward_only_reads_what_the_forward_saved(S):
+    """A second backward over the same saved forward finds what the first one found."""
+    m = _block(64, S, 3)
+    x = torch.randn(40, 19, 64, device="cuda").requires_grad_()
+    y = _run(m, x)
+    ps = [x] + list(m.parameters())
+    g = torch.randn_like(x)
+    saved = [t.clone() for t in y.grad_fn.saved_tensors]
+    ref = torch.autograd.grad(y, ps, g, retain_graph=True)
+    for a, b in zip(y.grad_fn.saved_tensors, saved):
+        assert torch.equal(a, b)
+    again = torch.autograd.grad(y, ps, g)
+    for a, b in zip(again, ref):
         assert torch.equal(a, b)
