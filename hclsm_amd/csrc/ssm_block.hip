@@ -320,7 +320,7 @@ __global__ void __launch_bounds__(256) block_reduce_kernel(RedGroup rg) {
 
 // ------------------------------------------------------------------------------------ LayerNorm, backward
 constexpr int LB_Q = 4;        // float4 units per lane: rows of up to 1024
-// gx = g + LN'(gu); per workgroup the partial sums of ggamma = sum gu xhat and gbeta = sum gu: part[block][2][D].
+// gx = g + LN'(gu) (gx nullable); per workgroup the partial sums of ggamma = sum gu xhat and gbeta = sum gu: part[block][2][D].
 __global__ void __launch_bounds__(256)
 block_ln_bwd_kernel(const float* __restrict__ x, const float* __restrict__ gu, const float* __restrict__ g,
                     const float* __restrict__ gamma, float* __restrict__ gx, float* __restrict__ part, int M, int D,
@@ -381,7 +381,7 @@ block_ln_bwd_kernel(const float* __restrict__ x, const float* __restrict__ gu, c
 #pragma unroll
     for (int q = 0; q < LB_Q; ++q) {
       const int u = lane + 64 * q;
-      if (u < nu)
+      if (u < nu && gx != nullptr)
         op[u] = make_float4(gv[q].x + rstd * (uv[q].x - a - xv[q].x * b), gv[q].y + rstd * (uv[q].y - a - xv[q].y * b),
                             gv[q].z + rstd * (uv[q].z - a - xv[q].z * b), gv[q].w + rstd * (uv[q].w - a - xv[q].w * b));
     }
@@ -421,7 +421,7 @@ block_gate_bwd_kernel(const uint32_t* __restrict__ gy, const uint32_t* __restric
 // --------------------------------------------------------------------------------------------- layouts
 struct BlkLayout {   // byte offsets; save: what the backward reads, scratch: the backward's own
   size_t u, z, gate, dt, b, c, y, y_pre, w, wt, ck, save;
-  size_t gy, gys, gz0, gdt, gbc, gg, gz, gu, part, lnp, scan, scratch;
+  size_t gy, gys, gz0, gdt, gbc, gg, gz, gu, part, lnp, ga, scan, scratch;
   int64_t R, part_ld;
   int splits, rows_per, ln_blocks;
   bool group, pair16;
@@ -464,6 +464,7 @@ static int blk_layout(int64_t N, int64_t T, int64_t d, int64_t di, int64_t S, bo
   L->part = take((size_t)L->splits * L->part_ld * 4);
   L->ln_blocks = (int)((R + 15) / 16 < 256 ? (R + 15) / 16 : 256);
   L->lnp = take((size_t)L->ln_blocks * 2 * d * 4);
+  L->ga = take(di * S * 4);
   L->scan = take(scan_ws - ck_bytes);
   L->scratch = o;
   return 0;
@@ -596,12 +597,14 @@ extern "C" int hclsm_ssm_block_backward(const HclsmBlockParams* P, const float* 
   BlkLayout L;
   int rc = blk_layout(batch, T, d, di, S, true, &L);
   if (rc) return rc;
-  if ((rc = blk_check(P, x, gx))) return rc;
-  if (!g || !G || !save || !scratch || !G->ln_w || !G->ln_b || !G->w_in || !G->w_gate || !G->w_dt || !G->b_dt || !G->w_b ||
-      !G->w_c || !G->a_log || !G->w_out)
-    return HCLSM_ERR_NULL;
+  if ((rc = blk_check(P, x, g))) return rc;
+  if (!G || !save || !scratch) return HCLSM_ERR_NULL;
   if (save_bytes < (int64_t)L.save || scratch_bytes < (int64_t)L.scratch) return HCLSM_ERR_SHAPE;
-  if (((uintptr_t)save & 255) || ((uintptr_t)scratch & 255) || !al16p(g)) return HCLSM_ERR_UNSUPPORTED;
+  if (((uintptr_t)save & 255) || ((uintptr_t)scratch & 255) || !al16p(gx)) return HCLSM_ERR_UNSUPPORTED;
+  // what the wanted gradients need: gu (the LayerNorm's), gz, the scan's backward
+  const bool need_u = gx || G->ln_w || G->ln_b, need_z = need_u || G->w_in;
+  const bool need_scan = need_z || G->w_gate || G->w_dt || G->b_dt || G->w_b || G->w_c || G->a_log;
+  float* gA = G->a_log ? G->a_log : reinterpret_cast<float*>(reinterpret_cast<char*>(scratch) + L.ga);
   hipStream_t st = (hipStream_t)stream;
   const char* s = reinterpret_cast<const char*>(save);
   char* q = reinterpret_cast<char*>(scratch);
@@ -609,46 +612,52 @@ extern "C" int hclsm_ssm_block_backward(const HclsmBlockParams* P, const float* 
   uint16_t* gB = reinterpret_cast<uint16_t*>(q + L.gbc);
   uint16_t* gC = reinterpret_cast<uint16_t*>(q + L.gbc + up256(L.R * S * 2));
   GemmGroup gg = {};
-  gg.np = 1;
-  gg.p[0] = prob(di, q + L.gy, di, 0);
-  add_seg(gg.p[0], g, d, w.out_t, d, d, 1);
-  if ((rc = run_gemm(gg, L.R, st))) return rc;
-  if (L.group) {
-    BwdGate gate;
-    gate.gate = s + L.gate; gate.y_pre = s + L.y_pre; gate.g_gate = q + L.gg;
-    rc = scan_bwd_block(s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, q + L.gy, q + L.gz0, q + L.gdt, G->a_log, gB, gC,
-                        batch, T, di, S, HCLSM_BF16, gate, nullptr, q + L.scan, (int64_t)(L.scratch - L.scan), st);
-  } else {
-    const int64_t n2 = L.R * di / 2;
-    const int64_t nb = (n2 + 255) / 256;
-    hipLaunchKernelGGL(block_gate_bwd_kernel, dim3((unsigned)(nb < 4096 ? nb : 4096)), dim3(256), 0, st,
-                       (const uint32_t*)(q + L.gy), (const uint32_t*)(s + L.gate), (const uint32_t*)(s + L.y_pre),
-                       (uint32_t*)(q + L.gys), (uint32_t*)(q + L.gg), n2);
-    HCLSM_LAUNCH_CHECK();
-    rc = scan_bwd_block(s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, q + L.gys, q + L.gz0, q + L.gdt, G->a_log, gB, gC,
-                        batch, T, di, S, HCLSM_BF16, BwdGate(), reinterpret_cast<const float*>(s + L.ck), q + L.scan,
-                        (int64_t)(L.scratch - L.scan), st);
+  if (need_scan) {
+    gg.np = 1;
+    gg.p[0] = prob(di, q + L.gy, di, 0);
+    add_seg(gg.p[0], g, d, w.out_t, d, d, 1);
+    if ((rc = run_gemm(gg, L.R, st))) return rc;
+    if (L.group) {
+      BwdGate gate;
+      gate.gate = s + L.gate; gate.y_pre = s + L.y_pre; gate.g_gate = q + L.gg;
+      rc = scan_bwd_block(s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, q + L.gy, q + L.gz0, q + L.gdt, gA, gB, gC,
+                          batch, T, di, S, HCLSM_BF16, gate, nullptr, q + L.scan, (int64_t)(L.scratch - L.scan), st);
+    } else {
+      const int64_t n2 = L.R * di / 2;
+      const int64_t nb = (n2 + 255) / 256;
+      hipLaunchKernelGGL(block_gate_bwd_kernel, dim3((unsigned)(nb < 4096 ? nb : 4096)), dim3(256), 0, st,
+                         (const uint32_t*)(q + L.gy), (const uint32_t*)(s + L.gate), (const uint32_t*)(s + L.y_pre),
+                         (uint32_t*)(q + L.gys), (uint32_t*)(q + L.gg), n2);
+      HCLSM_LAUNCH_CHECK();
+      rc = scan_bwd_block(s + L.z, s + L.dt, P->a_log, s + L.b, s + L.c, q + L.gys, q + L.gz0, q + L.gdt, gA, gB, gC,
+                          batch, T, di, S, HCLSM_BF16, BwdGate(), reinterpret_cast<const float*>(s + L.ck), q + L.scan,
+                          (int64_t)(L.scratch - L.scan), st);
+    }
+    if (rc) return rc;
   }
-  if (rc) return rc;
-  gg = {};
-  gg.np = 1;
-  gg.p[0] = prob(di, q + L.gz, di, 0);
-  add_seg(gg.p[0], q + L.gdt, di, w.dt_t, di, di);
-  add_seg(gg.p[0], gB, S, w.bc_t, 2 * S, S);
-  add_seg(gg.p[0], gC, S, w.bc_t + S, 2 * S, S);
-  gg.p[0].add = q + L.gz0; gg.p[0].ldadd = di;
-  if ((rc = run_gemm(gg, L.R, st))) return rc;
-  gg = {};
-  gg.np = 1;
-  gg.p[0] = prob(d, q + L.gu, d, 1);
-  add_seg(gg.p[0], q + L.gz, di, w.in_t, di, di);
-  add_seg(gg.p[0], q + L.gg, di, w.gate_t, di, di);
-  if ((rc = run_gemm(gg, L.R, st))) return rc;
+  if (need_z) {
+    gg = {};
+    gg.np = 1;
+    gg.p[0] = prob(di, q + L.gz, di, 0);
+    add_seg(gg.p[0], q + L.gdt, di, w.dt_t, di, di);
+    add_seg(gg.p[0], gB, S, w.bc_t, 2 * S, S);
+    add_seg(gg.p[0], gC, S, w.bc_t + S, 2 * S, S);
+    gg.p[0].add = q + L.gz0; gg.p[0].ldadd = di;
+    if ((rc = run_gemm(gg, L.R, st))) return rc;
+  }
   float* lnp = reinterpret_cast<float*>(q + L.lnp);
-  hipLaunchKernelGGL(block_ln_bwd_kernel, dim3((unsigned)L.ln_blocks), dim3(256), 0, st, x, (const float*)(q + L.gu), g,
-                     P->ln_w, gx, lnp, (int)L.R, (int)d, 1e-5f);
-  HCLSM_LAUNCH_CHECK();
-  // weight gradients
+  if (need_u) {
+    gg = {};
+    gg.np = 1;
+    gg.p[0] = prob(d, q + L.gu, d, 1);
+    add_seg(gg.p[0], q + L.gz, di, w.in_t, di, di);
+    add_seg(gg.p[0], q + L.gg, di, w.gate_t, di, di);
+    if ((rc = run_gemm(gg, L.R, st))) return rc;
+    hipLaunchKernelGGL(block_ln_bwd_kernel, dim3((unsigned)L.ln_blocks), dim3(256), 0, st, x, (const float*)(q + L.gu), g,
+                       P->ln_w, gx, lnp, (int)L.R, (int)d, 1e-5f);
+    HCLSM_LAUNCH_CHECK();
+  }
+  // weight gradients: those that are wanted (the bias's alone: the first column tile of its matrix)
   WgGroup wg = {};
   wg.M = (int)L.R; wg.rows_per = L.rows_per; wg.splits = L.splits; wg.part_ld = L.part_ld;
   wg.part = reinterpret_cast<float*>(q + L.part);
@@ -656,29 +665,35 @@ extern "C" int hclsm_ssm_block_backward(const HclsmBlockParams* P, const float* 
   int tiles = 0, rblk = 0;
   int64_t off = 0;
   auto red = [&](const float* src, int64_t ld, int n, float* dst, int64_t cnt) {
+    if (!dst) return;
     rg.s[rg.ns++] = RedSeg{src, ld, n, dst, (int)cnt, rblk};
     rblk += (int)((cnt + 63) / 64);
   };
-  auto wgrad = [&](const void* ga, int64_t N, int g_f32, const void* xa, int64_t K, float* dst) {
-    const int tx = (int)((K + 63) / 64);
-    wg.p[wg.np++] = WgProb{ga, N, g_f32, (int)N, (const uint16_t*)xa, K, (int)K, tx, off, -1, tiles};
-    tiles += tx * (int)((N + 63) / 64);
-    red(wg.part + off, L.part_ld, L.splits, dst, N * K);
+  auto wgrad = [&](const void* ga, int64_t N, int g_f32, const void* xa, int64_t K, float* dst, float* bias) {
+    if (dst || bias) {
+      const int tx = dst ? (int)((K + 63) / 64) : 1;
+      wg.p[wg.np++] = WgProb{ga, N, g_f32, (int)N, (const uint16_t*)xa, K, (int)K, tx, off, bias ? L.part_ld - di : -1, tiles};
+      tiles += tx * (int)((N + 63) / 64);
+      red(wg.part + off, L.part_ld, L.splits, dst, N * K);
+      red(wg.part + L.part_ld - di, L.part_ld, L.splits, bias, N);
+    }
     off += N * K;
   };
-  wgrad(q + L.gdt, di, 0, s + L.z, di, G->w_dt);
-  wg.p[0].bias_off = L.part_ld - di;
-  red(wg.part + wg.p[0].bias_off, L.part_ld, L.splits, G->b_dt, di);
-  wgrad(q + L.gz, di, 0, s + L.u, d, G->w_in);
-  wgrad(q + L.gg, di, 0, s + L.u, d, G->w_gate);
-  wgrad(g, d, 1, s + L.y, di, G->w_out);
-  wgrad(gB, S, 0, s + L.z, di, G->w_b);
-  wgrad(gC, S, 0, s + L.z, di, G->w_c);
+  wgrad(q + L.gdt, di, 0, s + L.z, di, G->w_dt, G->b_dt);
+  wgrad(q + L.gz, di, 0, s + L.u, d, G->w_in, nullptr);
+  wgrad(q + L.gg, di, 0, s + L.u, d, G->w_gate, nullptr);
+  wgrad(g, d, 1, s + L.y, di, G->w_out, nullptr);
+  wgrad(gB, S, 0, s + L.z, di, G->w_b, nullptr);
+  wgrad(gC, S, 0, s + L.z, di, G->w_c, nullptr);
   red(lnp, 2 * d, L.ln_blocks, G->ln_w, d);
   red(lnp + d, 2 * d, L.ln_blocks, G->ln_b, d);
-  hipLaunchKernelGGL(block_wgrad_kernel, dim3((unsigned)(tiles * L.splits)), dim3(256), 0, st, wg);
-  HCLSM_LAUNCH_CHECK();
-  hipLaunchKernelGGL(block_reduce_kernel, dim3((unsigned)rblk), dim3(256), 0, st, rg);
-  HCLSM_LAUNCH_CHECK();
+  if (wg.np) {
+    hipLaunchKernelGGL(block_wgrad_kernel, dim3((unsigned)(tiles * L.splits)), dim3(256), 0, st, wg);
+    HCLSM_LAUNCH_CHECK();
+  }
+  if (rg.ns) {
+    hipLaunchKernelGGL(block_reduce_kernel, dim3((unsigned)rblk), dim3(256), 0, st, rg);
+    HCLSM_LAUNCH_CHECK();
+  }
   return 0;
 }

@@ -21,7 +21,7 @@ class _Ptrs(ctypes.Structure):
 
 
 def _ptrs(tensors) -> _Ptrs:
-    return _Ptrs(*(t.data_ptr() for t in tensors))
+    return _Ptrs(*(None if t is None else t.data_ptr() for t in tensors))
 
 
 def _plain_linear(m, bias: bool) -> bool:
@@ -105,15 +105,15 @@ class _Block(torch.autograd.Function):
         g = _aligned(g.to(torch.float32))
         L = _lib.lib()
         scratch = torch.empty(int(L.hclsm_ssm_block_scratch(N, T, d, di, S)), dtype=torch.uint8, device=x.device)
-        gx = torch.empty_like(x)
-        grads = [torch.empty_like(p) for p in ps]
+        need = ctx.needs_input_grad               # (x, save, parameters): the others are not formed
+        gx = torch.empty_like(x) if need[0] else None
+        grads = [torch.empty_like(p) if n else None for p, n in zip(ps, need[2:])]
         st, sg = _ptrs(ps), _ptrs(grads)
-        rc = L.hclsm_ssm_block_backward(ctypes.byref(st), x.data_ptr(), g.data_ptr(), gx.data_ptr(), ctypes.byref(sg), N, T,
+        rc = L.hclsm_ssm_block_backward(ctypes.byref(st), x.data_ptr(), g.data_ptr(), _lib.ptr(gx), ctypes.byref(sg), N, T,
                                         d, di, S, save.data_ptr(), save.numel(), scratch.data_ptr(), scratch.numel(),
                                         _lib.stream_of(x))
         _lib.check(rc, "hclsm_ssm_block_backward")
-        need = ctx.needs_input_grad
-        return (gx if need[0] else None, None, *(v if n else None for v, n in zip(grads, need[2:])))
+        return (gx, None, *grads)
 
 
 def ssm_block(m, x):

@@ -156,8 +156,9 @@ int hclsm_ssm_scan_bwd_ckpt(const void* x, const void* dt, const float* A_log, c
  *   z = u w_in^T, gate = u w_gate^T, dt = z w_dt^T + b_dt, B = z w_b^T, C = z w_c^T (eps 1e-5).
  *   save:    hclsm_ssm_block_save bytes (256-byte aligned): intermediates; with train != 0 also what the backward reads.
  *   scratch: hclsm_ssm_block_scratch bytes (256-byte aligned), backward only.
- *   The backward takes the gradient g of out (fp32) and writes gx (x's, the residual included) and every parameter's
- *   gradient (fp32, overwritten).  save must hold what a forward with train != 0 left for the same inputs.
+ *   The backward takes the gradient g of out (fp32) and writes gx (x's, the residual included) and the parameters'
+ *   gradients (fp32, overwritten).  A null gx or member of grads is not formed, nor what only it needs.  save must hold
+ *   what a forward with train != 0 left for the same inputs.
  *   It only reads save: backward calls on several streams may share one, each with a scratch of its own.
  * Limits: d_model, d_inner and d_state multiples of 8, d_model <= 1024, d_inner <= 4096, d_state 16 or 24 .. 128 (64 at
  *   most where not a multiple of 16), batch * T <= 2^24, batch * T * d_inner < 2^30; HCLSM_ERR_UNSUPPORTED elsewhere.

@@ -74,3 +74,48 @@ def test_the_backward_only_reads_what_the_forward_saved(S):
     again = torch.autograd.grad(y, ps, g)
     for a, b in zip(again, ref):
         assert torch.equal(a, b)
+
+
+_PARAMS = {"norm.weight": "ln_w", "norm.bias": "ln_b", "in_proj.weight": "w_in", "gate_proj.weight": "w_gate",
+           "dt_proj.weight": "w_dt", "dt_proj.bias": "b_dt", "B_proj.weight": "w_b", "C_proj.weight": "w_c",
+           "A_log": "a_log", "out_proj.weight": "w_out"}
+
+
+@pytest.mark.parametrize("S", [16, 48])
+@pytest.mark.parametrize("wanted", [["x"], *([n] for n in _PARAMS), ["x", "A_log"], ["in_proj.weight", "dt_proj.bias"],
+                                    [n for n in _PARAMS if n != "dt_proj.weight"]])
+def test_only_the_wanted_gradients_are_formed(S, wanted, monkeypatch):
+    """Frozen inputs and parameters reach the library as null pointers; the others' gradients do not change."""
+    from hclsm_amd import _lib
+    from hclsm_amd.kernels import ssm_block
+    m = _block(72, S, 4)                                     # widths past one tile
+    x = torch.randn(5, 11, 72, device="cuda").requires_grad_()
+    g = torch.randn_like(x)
+    names = {"x": x, **dict(m.named_parameters())}
+    ref = dict(zip(names, torch.autograd.grad(_run(m, x), list(names.values()), g)))
+    for n, t in names.items():
+        t.requires_grad_(n in wanted)
+    seen = []
+
+    class Recorder:
+        def __getattr__(self, name):
+            fn = getattr(_lib.lib(), name)
+            if name != "hclsm_ssm_block_backward":
+                return fn
+
+            def call(*a):
+                sg = a[4]._obj
+                seen.append({"x": a[3], **{n: getattr(sg, c) for n, c in _PARAMS.items()}})
+                return fn(*a)
+            return call
+
+    class Lib:
+        def __getattr__(self, name):
+            return (lambda: Recorder()) if name == "lib" else getattr(_lib, name)
+
+    monkeypatch.setattr(ssm_block, "_lib", Lib())
+    got = torch.autograd.grad(_run(m, x), [names[n] for n in wanted], g)
+    for n, v in zip(wanted, got):
+        assert torch.equal(v, ref[n]), n
+    assert len(seen) == 1
+    assert {n for n, p in seen[0].items() if p} == set(wanted)
