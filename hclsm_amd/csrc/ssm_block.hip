@@ -597,10 +597,11 @@ extern "C" int hclsm_ssm_block_backward(const HclsmBlockParams* P, const float* 
   BlkLayout L;
   int rc = blk_layout(batch, T, d, di, S, true, &L);
   if (rc) return rc;
-  if ((rc = blk_check(P, x, g))) return rc;
-  if (!G || !save || !scratch) return HCLSM_ERR_NULL;
+  if (!P || !P->ln_w || !P->a_log || !x || !g || !G || !save || !scratch) return HCLSM_ERR_NULL;
   if (save_bytes < (int64_t)L.save || scratch_bytes < (int64_t)L.scratch) return HCLSM_ERR_SHAPE;
-  if (((uintptr_t)save & 255) || ((uintptr_t)scratch & 255) || !al16p(gx)) return HCLSM_ERR_UNSUPPORTED;
+  if (((uintptr_t)save & 255) || ((uintptr_t)scratch & 255) || !al16p(x) || !al16p(g) || !al16p(gx) || !al16p(P->ln_w) ||
+      !al16p(P->a_log))
+    return HCLSM_ERR_UNSUPPORTED;
   // what the wanted gradients need: gu (the LayerNorm's), gz, the scan's backward
   const bool need_u = gx || G->ln_w || G->ln_b, need_z = need_u || G->w_in;
   const bool need_scan = need_z || G->w_gate || G->w_dt || G->b_dt || G->w_b || G->w_c || G->a_log;

@@ -24,6 +24,11 @@ def _ptrs(tensors) -> _Ptrs:
     return _Ptrs(*(None if t is None else t.data_ptr() for t in tensors))
 
 
+def _shapes(d: int, di: int, S: int) -> tuple:
+    """The parameters' shapes in _NAMES order."""
+    return (d,), (d,), (di, d), (di, d), (di, di), (di,), (S, di), (S, di), (di, S), (d, di)
+
+
 def _plain_linear(m, bias: bool) -> bool:
     return type(m) is nn.Linear and (m.bias is not None) == bias and _no_hooks(m)
 
@@ -59,8 +64,7 @@ def block_params(m, x):
            not p.is_contiguous() for p in ps):
         return None
     d, di, S = x.shape[2], m.A_log.shape[0], m.A_log.shape[1]
-    want = ((d,), (d,), (di, d), (di, d), (di, di), (di,), (S, di), (S, di), (di, S), (d, di))
-    if any(tuple(p.shape) != s for p, s in zip(ps, want)):
+    if any(tuple(p.shape) != s for p, s in zip(ps, _shapes(d, di, S))):
         return None
     return ps
 
@@ -92,23 +96,22 @@ class _Block(torch.autograd.Function):
     def forward(ctx, x, save, *ps):
         out, rc = _forward(x, ps, save, True)
         _lib.check(rc, "hclsm_ssm_block_forward")
-        ctx.save_for_backward(x, save, *ps)
+        ctx.save_for_backward(x, save, ps[0], ps[8])   # (the backward's other parameters are in save, rounded)
         return out
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, g):
-        x, save, *ps = ctx.saved_tensors
-        x, save, ps = _aligned(x), _aligned(save, 256), [_aligned(p) for p in ps]
+        x, save, ln_w, a_log = (_aligned(t, 256 if t.dtype == torch.uint8 else 16) for t in ctx.saved_tensors)
         N, T, d = x.shape
-        di, S = ps[8].shape
+        di, S = a_log.shape
         g = _aligned(g.to(torch.float32))
         L = _lib.lib()
         scratch = torch.empty(int(L.hclsm_ssm_block_scratch(N, T, d, di, S)), dtype=torch.uint8, device=x.device)
         need = ctx.needs_input_grad               # (x, save, parameters): the others are not formed
         gx = torch.empty_like(x) if need[0] else None
-        grads = [torch.empty_like(p) if n else None for p, n in zip(ps, need[2:])]
-        st, sg = _ptrs(ps), _ptrs(grads)
+        grads = [torch.empty(s, dtype=x.dtype, device=x.device) if n else None for s, n in zip(_shapes(d, di, S), need[2:])]
+        st, sg = _Ptrs(ln_w=ln_w.data_ptr(), a_log=a_log.data_ptr()), _ptrs(grads)
         rc = L.hclsm_ssm_block_backward(ctypes.byref(st), x.data_ptr(), g.data_ptr(), _lib.ptr(gx), ctypes.byref(sg), N, T,
                                         d, di, S, save.data_ptr(), save.numel(), scratch.data_ptr(), scratch.numel(),
                                         _lib.stream_of(x))

@@ -159,7 +159,8 @@ int hclsm_ssm_scan_bwd_ckpt(const void* x, const void* dt, const float* A_log, c
  *   The backward takes the gradient g of out (fp32) and writes gx (x's, the residual included) and the parameters'
  *   gradients (fp32, overwritten).  A null gx or member of grads is not formed, nor what only it needs.  save must hold
  *   what a forward with train != 0 left for the same inputs.
- *   It only reads save: backward calls on several streams may share one, each with a scratch of its own.
+ *   Of params it reads ln_w and a_log (the matrices are in save, as the forward saw them); the others may be null or have
+ *   changed.  It only reads save: backward calls on several streams may share one, each with a scratch of its own.
  * Limits: d_model, d_inner and d_state multiples of 8, d_model <= 1024, d_inner <= 4096, d_state 16 or 24 .. 128 (64 at
  *   most where not a multiple of 16), batch * T <= 2^24, batch * T * d_inner < 2^30; HCLSM_ERR_UNSUPPORTED elsewhere.
  * Replaces: SimplifiedSSMBlock.forward (hclsm/dynamics/level0_ssm.py:58-107) and its autograd under bf16 autocast.

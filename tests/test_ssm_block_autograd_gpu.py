@@ -119,3 +119,29 @@ def test_only_the_wanted_gradients_are_formed(S, wanted, monkeypatch):
         assert torch.equal(v, ref[n]), n
     assert len(seen) == 1
     assert {n for n, p in seen[0].items() if p} == set(wanted)
+
+
+@pytest.mark.parametrize("S", [16, 48])
+def test_parameters_changed_before_the_backward(S):
+    """Matrices that the forward rounded to bf16 may change afterwards (a step of one loss before the backward of the
+    next, as with the module's ops); those that the backward reads itself may not."""
+    m = _block(64, S, 5)
+    x = torch.randn(3, 9, 64, device="cuda").requires_grad_()
+    g = torch.randn_like(x)
+    ps = [x] + list(m.parameters())
+    ref = torch.autograd.grad(_run(m, x), ps, g)
+    kept = {n: p.detach().clone() for n, p in m.named_parameters()}
+    y = _run(m, x)
+    with torch.no_grad():
+        for n, p in m.named_parameters():
+            if n not in ("norm.weight", "A_log"):
+                p.add_(1.0)
+    for a, b in zip(torch.autograd.grad(y, ps, g), ref):
+        assert torch.equal(a, b)
+    for name in ("norm.weight", "A_log"):
+        m.load_state_dict(kept)
+        y = _run(m, x)
+        with torch.no_grad():
+            m.get_parameter(name).add_(1.0)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(y, ps, g)
