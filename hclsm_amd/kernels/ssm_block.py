@@ -34,7 +34,9 @@ def _plain_linear(m, bias: bool) -> bool:
 
 
 def _no_hooks(m) -> bool:
-    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+    """Nothing is attached to the submodule: no hook, and no forward of the instance's own (as wrapping libraries set)."""
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or
+                "forward" in m.__dict__)
 
 
 def block_params(m, x):

@@ -145,3 +145,18 @@ def test_parameters_changed_before_the_backward(S):
             m.get_parameter(name).add_(1.0)
         with pytest.raises(RuntimeError, match="modified by an inplace operation"):
             torch.autograd.grad(y, ps, g)
+
+
+def test_a_submodules_own_forward_is_called():
+    """Libraries that wrap modules set `forward` on the instance: the module's ops run it."""
+    m = _block(64, 32, 6)
+    x = torch.randn(2, 5, 64, device="cuda")
+    with torch.autocast("cuda", dtype=torch.bfloat16), torch.no_grad():
+        plain = m(x)
+        for name in ("norm", "B_proj", "out_proj"):
+            sub, seen = getattr(m, name), []
+            sub.forward = lambda *a, f=type(sub).forward, sub=sub: seen.append(1) or f(sub, *a)
+            y = m(x)
+            del sub.forward
+            assert seen or name == "out_proj"      # (the module reads out_proj's weight itself)
+            assert (y - plain).norm() <= 2e-2 * plain.norm()
