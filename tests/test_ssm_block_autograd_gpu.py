@@ -1,12 +1,12 @@
 """The fused Level-0 block inside a larger autograd graph: incoming gradients and saved tensors at any address, the saved
-forward left as it is."""
+forward left as it is; and beside the module's own ops."""
 
 from __future__ import annotations
 
 import pytest
 import torch
 
-from test_ssm_block_gpu import _block
+from test_ssm_block_gpu import _block, _exact, _rel
 
 pytestmark = pytest.mark.gpu
 
@@ -160,3 +160,50 @@ def test_a_submodules_own_forward_is_called():
             del sub.forward
             assert seen or name == "out_proj"      # (the module reads out_proj's weight itself)
             assert (y - plain).norm() <= 2e-2 * plain.norm()
+
+
+def _both_ways(m, x, g):
+    """Output and gradients of the fused block and of the module's ops, and the same in float64."""
+    ps = [x] + list(m.parameters())
+    out = []
+    for hooked in (False, True):
+        h = m.B_proj.register_forward_hook(lambda mod, i, o: None) if hooked else None    # keeps the module's ops
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(x)
+        if h:
+            h.remove()
+        assert (type(y.grad_fn).__name__ == "_BlockBackward") != hooked
+        out.append((y.detach(), *torch.autograd.grad(y, ps, g)))
+    ye, ge = _exact(m, x, g)
+    return out, (ye, *ge.values())
+
+
+@pytest.mark.parametrize("N,T,d,S,expand", [
+    (70, 16, 192, 48, 2), (64, 33, 128, 16, 2), (40, 13, 128, 32, 2), (20, 17, 96, 128, 3), (300, 16, 192, 48, 2)])
+def test_no_further_from_float64_than_the_modules_ops(N, T, d, S, expand):
+    """The fused block makes a part of the module's roundings: its errors are no larger.  The two share the roundings
+    that weigh most (operands, the inputs of the scan), so their errors differ little; a tenth is left to chance."""
+    m = _block(d, S, N + S, expand)
+    gen = torch.Generator("cuda").manual_seed(N)
+    x = torch.randn(N, T, d, generator=gen, device="cuda").requires_grad_()
+    g = torch.randn(N, T, d, generator=gen, device="cuda")
+    (fused, module), exact = _both_ways(m, x, g)
+    for name, a, b, e in zip(["y", "x"] + [n for n, _ in m.named_parameters()], fused, module, exact):
+        assert _rel(a, e) <= 1.1 * _rel(b, e), (name, _rel(a, e), _rel(b, e))
+
+
+@pytest.mark.parametrize("d,S", [(64, 72), (64, 8), (36, 32), (64, 20)])
+def test_widths_that_keep_the_modules_ops(d, S):
+    """d_state past 64 that is no multiple of 16, below 16, or widths that are no multiples of 8."""
+    from hclsm_amd.kernels.ssm_block import ssm_block
+    m = _block(d, S, 8)
+    x = torch.randn(3, 9, d, device="cuda").requires_grad_()
+    g = torch.randn_like(x)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert ssm_block(m, x) is None
+        y = m(x)
+    grads = torch.autograd.grad(y, [x] + list(m.parameters()), g)
+    ye, ge = _exact(m, x, g)
+    assert _rel(y, ye) <= 2e-2
+    for v, n in zip(grads, ge):
+        assert _rel(v, ge[n]) <= 6e-2, n

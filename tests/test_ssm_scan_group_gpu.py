@@ -21,7 +21,8 @@ def _np(t):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("N,T,Dn,S", [
-    (1, 1, 1, 16),         # smallest, one group pair
+    (1, 1, 1, 16),         # d_state 16: one lane per channel
+    (1, 1, 1, 24),         # smallest of the state groups
     (2, 3, 63, 24),        # T below the chunk, a group count that does not divide it
     (3, 4, 64, 32),
     (2, 5, 65, 48),        # one past the chunk and the channel block
