@@ -25,7 +25,8 @@ __device__ __forceinline__ float scan_dt(float v) {
 }
 
 // Forward scan with a channel's states split over the waves of a workgroup (ssm_scan_group.hip): fp32 or bf16,
-// d_state a multiple of 8 from 24 (fp32 also 16) to 128.  HCLSM_ERR_UNSUPPORTED where it does not apply (the caller runs the generic kernel).
+// d_state a multiple of 8 from 24 to 128.  HCLSM_ERR_UNSUPPORTED where it does not apply (the caller runs the generic
+// kernel).
 int scan_fwd_group(int mode, const void* x, const void* dt, const float* A_log, const void* B, const void* C,
                    const float* Dskip, void* y, float* h_final, int64_t batch, int64_t T, int64_t Dn, int64_t S,
                    int dtype, hipStream_t st, ScanEpi epi);

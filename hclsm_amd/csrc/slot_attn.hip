@@ -1975,26 +1975,24 @@ core_update_t_kernel(const typename MM<DT>::T* __restrict__ P, int64_t Mp, const
   float cs = 0.f;
 #pragma unroll 2
   for (int m0 = 0; m0 < (int)Mp; m0 += 32) {
-    {
-      typename A::Op bv = A::load(pv + m0 + 8 * g);
-      if (m0 + 32 > a.M) {   // tokens past M: v rows are not initialised, zero them
-        TT e[8];
-        *reinterpret_cast<uint4*>(e) = __builtin_bit_cast(uint4, bv);
+    typename A::Op bv = A::load(pv + m0 + 8 * g);
+    if (m0 + 32 > a.M) {   // tokens past M: v rows are not initialised, zero them
+      TT e[8];
+      *reinterpret_cast<uint4*>(e) = __builtin_bit_cast(uint4, bv);
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (m0 + 8 * g + i >= a.M) e[i] = A::fromf(0.f);
-        bv = __builtin_bit_cast(typename A::Op, *reinterpret_cast<uint4*>(e));
-      }
-      if (renorm) {
-        TT e[8];
-        *reinterpret_cast<uint4*>(e) = __builtin_bit_cast(uint4, bv);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) cs += A::tof(e[i]);
-      }
-#pragma unroll
-      for (int nt = 0; nt < CORE_MAX_NT; ++nt)
-        if (nt < a.NT) acc[nt] = A::mfma(A::load(prow[nt] + m0 + 8 * g), bv, acc[nt]);
+      for (int i = 0; i < 8; ++i)
+        if (m0 + 8 * g + i >= a.M) e[i] = A::fromf(0.f);
+      bv = __builtin_bit_cast(typename A::Op, *reinterpret_cast<uint4*>(e));
     }
+    if (renorm) {
+      TT e[8];
+      *reinterpret_cast<uint4*>(e) = __builtin_bit_cast(uint4, bv);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) cs += A::tof(e[i]);
+    }
+#pragma unroll
+    for (int nt = 0; nt < CORE_MAX_NT; ++nt)
+      if (nt < a.NT) acc[nt] = A::mfma(A::load(prow[nt] + m0 + 8 * g), bv, acc[nt]);
   }
   cs = rows4_sum(cs);
   if (d >= a.D) return;

@@ -11,9 +11,9 @@
 //
 // What it replaces took 63 launches per step of a 1024 x 16 layer of width 192 (d_state 48): the weight gradients as
 // library GEMMs over 16384 rows without a row split (six of 98 us), ten elementwise passes for the gate, a cast per
-// weight and operand; the host needed 1.2 ms for them whatever the size.  Now 14 launches, 709 us of kernels against
-// 1522: scan backward 387, forward 88, six GEMM launches 109, weight gradients 63 (239 with a branch per load, which
-// left one load in flight), LayerNorm's backward 26, the rest 36.
+// weight and operand; the host needed 1.2 ms for them whatever the size.  Now 14 launches, 685 us of kernels against
+// 1522: scan backward 373, forward 81, six GEMM launches 108, weight gradients 60 (239 with a branch per load, which
+// left one load in flight), LayerNorm's backward 27, the rest 36.
 #include "internal.h"
 #include "mfma.h"
 #include "scan_common.h"
@@ -398,7 +398,7 @@ block_ln_bwd_kernel(const float* __restrict__ x, const float* __restrict__ gu, c
   }
 }
 
-// The gate's chain rule where the scan's backward does not take it: gy <- gy silu(gate) in place of nothing else's,
+// The gate's chain rule where the scan's backward does not take it (d_state 16): g_scan = gy silu(gate),
 // g_gate = gy y_pre silu'(gate).  Pairs of 16-bit elements.
 __global__ void __launch_bounds__(256)
 block_gate_bwd_kernel(const uint32_t* __restrict__ gy, const uint32_t* __restrict__ gate, const uint32_t* __restrict__ yp,

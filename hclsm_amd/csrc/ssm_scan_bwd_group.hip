@@ -15,9 +15,12 @@
 // up to three bf16 pieces; see ssm_scan_group.hip for non-finite values).  SG = 8: on the VALU.
 //
 // Bound by VALU issue (about 30 slots per state update: 6 for each of three forward evaluations, 10 for the reverse
-// step, 5 for the two sums across the wave) at 3 to 4 waves per SIMD.  Measured on MI355X, us per call with the tail
+// step, 5 for the two sums across the wave) with few waves to hide it: registers allow 4 per SIMD at 8 states a lane and
+// 3 at 16, LDS (160 KB a CU) workgroups of 12 waves at d_state 24, 32 and 48, 15, 14 and 16 at 40, 56 and 64 with 8 a
+// lane; 9, 10, 6, 7 and 8 at 48, 80, 96, 112 and 128 with 16.  16 a lane spills (40 registers, 72 with the gate; fp32 76
+// to 82), 8 a lane does not.  Measured on MI355X, us per call with the tail
 // launch (before: states padded to a power of two over 2 or 4 lanes of a wave, 44 KB of LDS per two waves):
-//   1024 x 16 x 384, S 48, bf16     701 -> 353 (block 804 -> 372)    512 x 16 x 512, S 64, fp32  472 -> 251
+//   1024 x 16 x 384, S 48, bf16     701 -> 352 (block 804 -> 383)    512 x 16 x 512, S 64, fp32  472 -> 251
 //   256 x 64 x 384, S 32, bf16      287 -> 223                       121 x 120 x 192, S 32, fp32 263 -> 179
 //   64 x 16 x 768, S 96, bf16 block 332 -> 125                       128 x 16 x 256, S 32, fp32 43.6 -> 28.3
 // Not kept: d_state 16 as two groups (1024 x 64 x 384: 416 -> 787), pointers instead of buffer resources (more registers),
@@ -447,23 +450,25 @@ int bwd_group(int mode, const void* x, const void* dt, const float* A_log, const
   if (mode == MODE_)                                                                                               \
     return launch_group<DT_, MODE_, SG_>(x, dt, A_log, B, C, Dskip, gy, gx, gdt, gate, ck, gbc, ga, gd, N, T, Dn, S, \
                                          parts, st);
-#define HCLSM_BG_M(DT_, SG_)                                                               \
-  HCLSM_BG(DT_, SG_, HCLSM_SCAN_RAW) HCLSM_BG(DT_, SG_, HCLSM_SCAN_MODEL)                  \
-  HCLSM_BG(DT_, SG_, HCLSM_SCAN_BLOCK) HCLSM_BG(DT_, SG_, BWD_BLOCK_GATE)
+#define HCLSM_BG_M(DT_, SG_) \
+  HCLSM_BG(DT_, SG_, HCLSM_SCAN_RAW) HCLSM_BG(DT_, SG_, HCLSM_SCAN_MODEL) HCLSM_BG(DT_, SG_, HCLSM_SCAN_BLOCK)
   int cus = 0;
   if (int rc = device_cus(&cus)) return rc;
-  // A CU has 16 wave slots at 8 states a lane (4 waves per SIMD) and 12 at 16 a lane.  Workgroups of S/8 waves that do
-  // not divide 16 leave slots empty, 4 of them at d_state 48, where S/16 = 3 waves divide 12: us 16 | 8 a lane in bf16,
-  // 1024 x 16 x 384: 353 | 407, block 372 | 499.  With few workgroups the slots are empty anyway, and fp32 has no matrix
-  // core to take the wider lane's products: 16 x 128 x 512 in fp32 262 | 182.  32 and 64 states fill the slots at 8 a
-  // lane; past 64 states 8 a lane would need more than 8 waves.
+  // 8 or 16 states a lane.  Past 64 states 8 a lane would need more than 8 waves.  The widths with a choice are 32, 48 and
+  // 64; forward and backward together in us, 8 | 16 a lane:
+  //   bf16 1024 x 16 x 384:  242 | 302   475 | 419   435 | 483     bf16 256 x 64 x 384:  281 | 432   533 | 526   499 | 654
+  //   bf16 32 x 64 x 384:    151 | 169   152 | 174   155 | 175     fp32 512 x 16 x 512:         304 | 360   317 | 383
+  // 16 a lane halves the waves and takes the rank-1 products off the VALU in bf16 (fp32 has no matrix core for them) but
+  // spills 40 to 72 registers: it gains on full grids at 48 alone, the width whose workgroups of S/8 waves do not divide
+  // the 16 wave slots that the registers of 8 a lane allow.  (Wave slots are not the whole reason: LDS leaves 12 of them
+  // in use at 32 and at 48.)
   const bool gaps = S % 16 == 0 && 16 % (S / 8) != 0;
   const bool wide = S > 8 * BG_MAX_WAVES || (dtype == HCLSM_BF16 && gaps && N * ((Dn + 63) / 64) >= 4 * (int64_t)cus);
   if (wide) {
-    if (dtype == HCLSM_BF16) { HCLSM_BG_M(HCLSM_BF16, 16) }
+    if (dtype == HCLSM_BF16) { HCLSM_BG_M(HCLSM_BF16, 16) HCLSM_BG(HCLSM_BF16, 16, BWD_BLOCK_GATE) }
     else { HCLSM_BG_M(HCLSM_F32, 16) }
   } else {
-    if (dtype == HCLSM_BF16) { HCLSM_BG_M(HCLSM_BF16, 8) }
+    if (dtype == HCLSM_BF16) { HCLSM_BG_M(HCLSM_BF16, 8) HCLSM_BG(HCLSM_BF16, 8, BWD_BLOCK_GATE) }
     else { HCLSM_BG_M(HCLSM_F32, 8) }
   }
 #undef HCLSM_BG_M

@@ -22,8 +22,8 @@
 // readout FMA), 6 on the VALU.  Measured on MI355X (us per launch; before: one to four lanes per channel, states
 // padded to a power of two, B / C through LDS; last: the slots at 1.75 ns each):
 //   128 x 16 x 256, S 32, fp32          15.6 ->   8.7   2.7     512 x 16 x 512, S 64, fp32   80.0 -> 61.9  43.0
-//   1024 x 16 x 384, S 48, bf16 block  246.3 ->  86.8  40.3     512 x 16 x 512, S 64, bf16   79.3 -> 58.0  35.9
-//   1024 x 64 x 384, S 32, bf16        183.7 -> 150.2 107.5     20 x 95 x 768, S 24, bf16    59.0 -> 34.1
+//   1024 x 16 x 384, S 48, bf16 block  246.3 ->  80.8  40.3     512 x 16 x 512, S 64, bf16   79.3 -> 53.9  35.9
+//   1024 x 64 x 384, S 32, bf16        183.7 -> 147.5 107.5     20 x 95 x 768, S 24, bf16    59.0 -> 34.1
 // Not kept: two channels per lane (1024 x 16 x 384 block 109 against 81, others equal or slower), 8-step chunks (equal),
 // B / C rows by vector loads a chunk ahead (172 registers: 10.7 against 8.6 at the first shape).
 #include "internal.h"

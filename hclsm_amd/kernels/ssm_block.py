@@ -1,6 +1,8 @@
 """A whole SimplifiedSSMBlock (hclsm/dynamics/level0_ssm.py:30-107) under a bf16 autocast on MI355X
-(libhclsm_amd.so: hclsm_ssm_block_forward / hclsm_ssm_block_backward): one library call each way, with the
-roundings of the module's ops (bf16 operands and intermediates, fp32 residual stream, parameters and gradients).
+(libhclsm_amd.so: hclsm_ssm_block_forward / hclsm_ssm_block_backward): one library call each way, with bf16 operands
+and intermediates where the module's ops have them, fp32 residual stream, parameters and gradients.  The output
+projection, the parts of z's gradient and the weight gradients, which the module's ops round to bf16 one by one, are
+summed in fp32, and every sum has its own order: results differ from the module's ops in bf16 roundings.
 """
 
 from __future__ import annotations
