@@ -20,7 +20,7 @@
 // lane; 9, 10, 6, 7 and 8 at 48, 80, 96, 112 and 128 with 16.  16 a lane spills (40 registers, 72 with the gate; fp32 76
 // to 82), 8 a lane does not.  Measured on MI355X, us per call with the tail
 // launch (before: states padded to a power of two over 2 or 4 lanes of a wave, 44 KB of LDS per two waves):
-//   1024 x 16 x 384, S 48, bf16     701 -> 352 (block 804 -> 383)    512 x 16 x 512, S 64, fp32  472 -> 251
+//   1024 x 16 x 384, S 48, bf16     701 -> 357 (block 804 -> 385)    512 x 16 x 512, S 64, fp32  472 -> 251
 //   256 x 64 x 384, S 32, bf16      287 -> 223                       121 x 120 x 192, S 32, fp32 263 -> 179
 //   64 x 16 x 768, S 96, bf16 block 332 -> 125                       128 x 16 x 256, S 32, fp32 43.6 -> 28.3
 // Not kept: d_state 16 as two groups (1024 x 64 x 384: 416 -> 787), pointers instead of buffer resources (more registers),
@@ -300,6 +300,10 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
           for (int e = 0; e < VL; ++e) red[i * 2 * S + S + s0 + off + e] = v[e];
         }
         asm volatile("" ::: "memory");   // the reverse steps recompute the gates (registers are the occupancy limit)
+        // the chunk's part of gA, in the places of hk's states as they are used up: four steps summed first keep the chain
+        // of additions over a walk short (error of gA_log against float64 at 512 x 16 x 512, S 64: 1.7e-7; step by step
+        // 2.4e-7, one partial per sequence 1.8e-7; 354.8 -> 356.8 us at 1024 x 16 x 384, S 48, else equal)
+        float gc[SG];
 #pragma unroll
         for (int i = K - 1; i >= 0; --i) {
           const int r = c * K + i;
@@ -323,7 +327,8 @@ ssm_scan_bwd_group_kernel(const typename Elem<DT>::T* __restrict__ x, const type
             gh[j] *= fast_exp2(dv * a2[j]);      // carried to step t-1
             const float garg = gh[j] * hp;
             gda2 = fmaf(garg, a2[j], gda2);
-            gA[j] = fmaf(garg, dv, gA[j]);
+            gc[j] = i == K - 1 ? garg * dv : fmaf(garg, dv, gc[j]);
+            if (i == 0) gA[j] += gc[j];
           }
           sQ[((i * 2 + 0) * NG + g) * 64 + l] = q;
           sQ[((i * 2 + 1) * NG + g) * 64 + l] = gda2;

@@ -73,3 +73,25 @@ def test_nonfinite_inputs_stay_in_their_channel(dtype, N):
                 assert torch.equal(got[name][keep], clean[name][keep]), (which, bad, name)
             rows = torch.arange(64, device="cuda") != 40
             assert torch.equal(got["A_log"][rows], clean["A_log"][rows])
+
+
+@pytest.mark.parametrize("N,T,Dn,S", [(512, 16, 512, 64), (1024, 16, 384, 48)])
+def test_gA_log_sums_over_a_walk(N, T, Dn, S):
+    """gA_log where a workgroup walks 4 to 8 sequences: the rounding of its sums.  An fp32 addition of random terms
+    rounds by 2.4e-8 (rms), a chain of k by 2.4e-8 sqrt(k / 2), and the terms themselves are good to 1.45e-7.  The walk's
+    chain is 32 sums of four steps at most: 1.75e-7 in all; step by step it is 128: 2.4e-7.  (One partial per sequence and
+    a chain of 32 of them: 1.9e-7.)"""
+    from hclsm_amd import _lib
+    from hclsm_amd.kernels.ssm_scan_bwd import scan_backward
+    d, gy = _case(N, T, Dn, S, torch.float32, "raw", N + S)
+    x, dt, A_log, B, C = (d[k].cuda() for k in ("x", "dt", "A_log", "B", "C"))
+    gy = gy.cuda()
+    got = scan_backward(x, dt, A_log, B, C, None, gy, _lib.SCAN_RAW)["A_log"].double()
+    al = A_log.double().requires_grad_()
+    A, h, loss = -torch.exp(al), torch.zeros(N, Dn, S, dtype=torch.float64, device="cuda"), 0.0
+    for t in range(T):
+        h = torch.exp(dt[:, t, :, None].double() * A) * h + (dt[:, t].double() * x[:, t].double())[..., None] * B[:, t, None].double()
+        loss = loss + ((h * C[:, t, None].double()).sum(-1) * gy[:, t].double()).sum()
+    want, = torch.autograd.grad(loss, al)
+    err = float((got - want).norm() / want.norm())
+    assert err <= 1.9e-7, f"{err:.3e}"
