@@ -31,14 +31,17 @@ def _shapes(d: int, di: int, S: int) -> tuple:
     return (d,), (d,), (di, d), (di, d), (di, di), (di,), (S, di), (S, di), (di, S), (d, di)
 
 
-def _plain_linear(m, bias: bool) -> bool:
-    return type(m) is nn.Linear and (m.bias is not None) == bias and _no_hooks(m)
-
-
-def _no_hooks(m) -> bool:
-    """Nothing is attached to the submodule: no hook, and no forward of the instance's own (as wrapping libraries set)."""
-    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or
-                "forward" in m.__dict__)
+def _params(m, cls):
+    """(weight, bias) of a submodule that is a plain cls to which nothing is attached (no hook, and no forward of the
+    instance's own, as wrapping libraries set), else (None, None).  What m.weight finds, an entry of the instance or
+    else a parameter, without the 0.5 us that the attribute of a module costs."""
+    if type(m) is not cls:
+        return None, None
+    d = m.__dict__
+    if "forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]:
+        return None, None
+    ps = d["_parameters"]
+    return d["weight"] if "weight" in d else ps.get("weight"), d["bias"] if "bias" in d else ps.get("bias")
 
 
 def block_params(m, x):
@@ -56,19 +59,22 @@ def block_params(m, x):
     if mm._global_forward_hooks or mm._global_forward_pre_hooks or mm._global_backward_hooks or mm._global_backward_pre_hooks:
         return None
     norm = m.norm
-    if type(norm) is not nn.LayerNorm or norm.eps != 1e-5 or norm.bias is None or not _no_hooks(norm):
+    ln_w, ln_b = _params(norm, nn.LayerNorm)
+    if ln_b is None or norm.eps != 1e-5:
         return None
-    if not (all(_plain_linear(p, False) for p in (m.in_proj, m.gate_proj, m.B_proj, m.C_proj, m.out_proj))
-            and _plain_linear(m.dt_proj, True)):
+    (w_in, b0), (w_gate, b1), (w_dt, b_dt), (w_b, b2), (w_c, b3), (w_out, b4) = [
+        _params(p, nn.Linear) for p in (m.in_proj, m.gate_proj, m.dt_proj, m.B_proj, m.C_proj, m.out_proj)]
+    if not (b0 is b1 is b2 is b3 is b4 is None):
         return None
-    ps = (norm.weight, norm.bias, m.in_proj.weight, m.gate_proj.weight, m.dt_proj.weight, m.dt_proj.bias,
-          m.B_proj.weight, m.C_proj.weight, m.A_log, m.out_proj.weight)
+    ps = (ln_w, ln_b, w_in, w_gate, w_dt, b_dt, w_b, w_c, m.A_log, w_out)    # (a None among them ends below)
     dev = x.device
     if any(type(p) not in (nn.Parameter, torch.Tensor) or p.dtype != torch.float32 or p.device != dev or
            not p.is_contiguous() for p in ps):
         return None
-    d, di, S = x.shape[2], m.A_log.shape[0], m.A_log.shape[1]
-    if any(tuple(p.shape) != s for p, s in zip(ps, _shapes(d, di, S))):
+    if ps[8].dim() != 2:
+        return None
+    d, (di, S) = x.shape[2], ps[8].shape
+    if any(p.shape != s for p, s in zip(ps, _shapes(d, di, S))):
         return None
     return ps
 
@@ -114,7 +120,7 @@ class _Block(torch.autograd.Function):
         scratch = torch.empty(int(L.hclsm_ssm_block_scratch(N, T, d, di, S)), dtype=torch.uint8, device=x.device)
         need = ctx.needs_input_grad               # (x, save, parameters): the others are not formed
         gx = torch.empty_like(x) if need[0] else None
-        grads = [torch.empty(s, dtype=x.dtype, device=x.device) if n else None for s, n in zip(_shapes(d, di, S), need[2:])]
+        grads = [x.new_empty(s) if n else None for s, n in zip(_shapes(d, di, S), need[2:])]
         st, sg = _Ptrs(ln_w=ln_w.data_ptr(), a_log=a_log.data_ptr()), _ptrs(grads)
         rc = L.hclsm_ssm_block_backward(ctypes.byref(st), x.data_ptr(), g.data_ptr(), _lib.ptr(gx), ctypes.byref(sg), N, T,
                                         d, di, S, save.data_ptr(), save.numel(), scratch.data_ptr(), scratch.numel(),
