@@ -11,9 +11,10 @@
 //
 // What it replaces took 63 launches per step of a 1024 x 16 layer of width 192 (d_state 48): the weight gradients as
 // library GEMMs over 16384 rows without a row split (six of 98 us), ten elementwise passes for the gate, a cast per
-// weight and operand; the host needed 1.2 ms for them whatever the size.  Now 14 launches, 685 us of kernels against
-// 1522: scan backward 373, forward 81, six GEMM launches 108, weight gradients 60 (239 with a branch per load, which
-// left one load in flight), LayerNorm's backward 27, the rest 36.
+// weight and operand, 2160 us in all; the host needed 1.1 to 1.3 ms for them whatever the size.  Now 14 launches and 683
+// us: scan backward 390, forward 85, six GEMM launches 107, weight gradients 62 (239 with a branch per load, which left
+// one load in flight), LayerNorm's backward 26, the rest 34 (each kernel in the trace; together 3% more than the call).
+// Smaller layers are bound by the host here too: 512 x 16, width 128, d_state 32, 1360 -> 315 us.
 #include "internal.h"
 #include "mfma.h"
 #include "scan_common.h"

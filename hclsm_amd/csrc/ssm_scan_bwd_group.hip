@@ -20,9 +20,9 @@
 // lane; 9, 10, 6, 7 and 8 at 48, 80, 96, 112 and 128 with 16.  16 a lane spills (40 registers, 72 with the gate; fp32 76
 // to 82), 8 a lane does not.  Measured on MI355X, us per call with the tail
 // launch (before: states padded to a power of two over 2 or 4 lanes of a wave, 44 KB of LDS per two waves):
-//   1024 x 16 x 384, S 48, bf16     701 -> 357 (block 804 -> 385)    512 x 16 x 512, S 64, fp32  472 -> 251
-//   256 x 64 x 384, S 32, bf16      287 -> 223                       121 x 120 x 192, S 32, fp32 263 -> 179
-//   64 x 16 x 768, S 96, bf16 block 332 -> 125                       128 x 16 x 256, S 32, fp32 43.6 -> 28.3
+//   1024 x 16 x 384, S 48, bf16     701 -> 356 (block 804 -> 377)    512 x 16 x 512, S 64, fp32  472 -> 251
+//   256 x 64 x 384, S 32, bf16      287 -> 226                       121 x 120 x 192, S 32, fp32 263 -> 179
+//   64 x 16 x 768, S 96, bf16 block 332 -> 126                       128 x 16 x 256, S 32, fp32 43.6 -> 28.9
 // Not kept: d_state 16 as two groups (1024 x 64 x 384: 416 -> 787), pointers instead of buffer resources (more registers),
 // the outputs' inputs requested before the reverse steps (13 registers more: one wave per SIMD less).
 #include "internal.h"
